@@ -1,4 +1,6 @@
-// gemm_f32.hip — fp32 GEMM on gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
+// gemm_f32.hip — fp32 GEMM on gfx950 matrix cores: every product through its
+// bf16 pieces (split_tile.hpp), with the fp32 MFMA for the data and strides
+// that path does not take.
 //
 // Entry points: omHipMatmul / MatmulTransB / MatmulTransA / BatchedMatmul /
 // BatchedMatmulTransB / GemmStridedBatched. They replace the reference's
@@ -9,6 +11,7 @@
 // (src/engine/om.engine.autograd.ixx:261-286).
 #include "omhip_internal.hpp"
 #include "mfma_f32_tile.hpp"
+#include "split_tile.hpp"
 #include "buffer_io.hpp"
 #include "gemm_f32.hpp"
 #include "../../include/omhip.h"
@@ -18,91 +21,6 @@
 #include <type_traits>
 
 namespace omhip {
-
-// Dense operand loader through range-checked buffer loads, 16-byte vectors
-// along the contiguous axis (element (r,k) at P[r*ld + k] when KMAJOR, at
-// P[k*ld + r] otherwise). A thread's byte offsets inside the tile are fixed
-// at init, rows past the matrix get kOOB (read as zeros), and each slice
-// re-bases the buffer view at the slice's first element with scalar
-// arithmetic: a whole slice is PER_T buffer loads and no vector ALU work.
-// Only the last, partial slice of a K range tests k per vector.
-// Host conditions (bufVecOk): the vector layout of DenseLoader (contiguous
-// axis, ld and base multiples of 4 floats) and every in-tile offset below
-// 2^30 bytes.
-template <bool KMAJOR, int R, int BK, int NT>
-struct BufVecLoader {
-    static constexpr int PER_T = R * BK / 4 / NT;
-    static_assert(R * BK % (NT * 4) == 0, "tile must split evenly over threads");
-    using Shape = LdsShape<KMAJOR, R, BK>;
-
-    const float* tile;   // element (r0, k = 0) of the operand
-    long long ld;
-    uint32_t voff[PER_T];
-    f32x4 v4[PER_T];
-
-    static __device__ __forceinline__ void coords(int e, int& r, int& k) {
-        if constexpr (KMAJOR) { r = e / (BK / 4); k = (e % (BK / 4)) * 4; }
-        else { k = e / (R / 4); r = (e % (R / 4)) * 4; }
-    }
-
-    __device__ void init(const float* p, long long ld_, int rows, int r0, int tid) {
-        ld = ld_;
-        tile = KMAJOR ? p + (long long)r0 * ld : p + r0;
-#pragma unroll
-        for (int i = 0; i < PER_T; ++i) {
-            int r, k;
-            coords(tid + i * NT, r, k);
-            voff[i] = (r0 + r < rows) ? (uint32_t)((KMAJOR ? r * ld + k : k * ld + r) * 4) : kOOB;
-        }
-    }
-
-    // FULL: the slice [k0, k0 + BK) lies inside [0, kEnd).
-    template <bool FULL>
-    __device__ void load(int k0, int kEnd, int tid) {
-        const auto rs = bufferRsrc(tile + (KMAJOR ? (long long)k0 : (long long)k0 * ld), kMaxBufferBytes);
-#pragma unroll
-        for (int i = 0; i < PER_T; ++i) {
-            uint32_t o = voff[i];
-            if constexpr (!FULL) {
-                int r, k;
-                coords(tid + i * NT, r, k);
-                if (k0 + k >= kEnd) o = kOOB;
-            }
-            v4[i] = bufLoad4(rs, o, 0);
-        }
-    }
-
-    __device__ void store(float* s, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER_T; ++i) {
-            int r, k;
-            coords(tid + i * NT, r, k);
-            float* dst = KMAJOR ? s + r * Shape::LD + k : s + k * Shape::LD + r;
-            *reinterpret_cast<f32x4*>(dst) = v4[i];
-        }
-    }
-};
-
-// The generic loader behind the same interface (any alignment, 64-bit
-// addressing, per-element bounds tests on every slice).
-template <bool KMAJOR, bool VEC, int R, int BK, int NT>
-struct DenseLoaderAdapter : DenseLoader<KMAJOR, VEC, R, BK, NT> {
-    using Base = DenseLoader<KMAJOR, VEC, R, BK, NT>;
-    __device__ void init(const float* p, long long ld, int rows, int r0, int) {
-        this->p = p; this->ld = ld; this->rows = rows; this->r0 = r0;
-    }
-    template <bool FULL>
-    __device__ void load(int k0, int kEnd, int tid) {
-        this->K = kEnd;
-        Base::load(k0, tid);
-    }
-};
-
-// Operand loader kinds: 0 generic scalar, 1 generic 16-byte vectors,
-// 2 buffer-view 16-byte vectors.
-template <bool KMAJOR, int LK, int R, int BK, int NT>
-using GemmLoader = std::conditional_t<LK == 2, BufVecLoader<KMAJOR, R, BK, NT>,
-                                      DenseLoaderAdapter<KMAJOR, LK == 1, R, BK, NT>>;
 
 // Split-K arrival of one piece of a tile. The piece's accumulators go to its
 // slot of ws in the tile's own register layout ([split][batch][tile] blocks of
@@ -193,24 +111,164 @@ __device__ __forceinline__ bool splitArrive(const GemmF32Params& p, f32x16 (&acc
     return true;
 }
 
-// One output tile (bid: the tile's linear index, batch, split) of C =
-// op(A) * op(B). BSUM (B stored [K, N]): the workgroups of the first row of
-// tiles also add B's columns over K, row after row from 0, into p.colSum (the
-// bias gradient of a Linear layer whose output gradient is B). GATE: each
-// element of C is kept where p.gate (same shape, row stride p.ldg) is > 0 and
-// set to 0 elsewhere (a ReLU's backward applied to the product).
-template <class Cfg, bool TA, bool TB, int LA, int LB, bool BSUM = false, bool GATE = false>
-__device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, float* smem, int bid, long long batch, int split) {
-    static_assert(!BSUM || !TB, "column sums of a B stored [K, N]");
-    constexpr bool A_KMAJOR = !TA;
-    constexpr bool B_KMAJOR = TB;
-    using SA = LdsShape<A_KMAJOR, Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<B_KMAJOR, Cfg::BN, Cfg::BK>;
-    constexpr int STAGE = SA::SIZE + SB::SIZE;   // floats per LDS buffer (A slice then B slice)
+// acc = op(A) * op(B) over [kBeg, kEnd) for one wave's WM x WN block at (m0, n0)
+// on the fp32 MFMA, its fragments read from memory element by element behind
+// bounds tests: any stride and alignment, no LDS. It recomputes the blocks
+// whose operands the pieces cannot carry, and serves strides beyond the buffer
+// views' range.
+template <class Cfg, bool TA, bool TB>
+__device__ __forceinline__ void plainProduct(const GemmF32Params& p, f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0, int n0,
+                                             long long batch, int kBeg, int kEnd, int lane) {
+    const int li = lane & 31, h = lane >> 5;
+    const float* A = p.A + batch * p.sA;
+    const float* B = p.B + batch * p.sB;
+#pragma unroll
+    for (int i = 0; i < Cfg::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < Cfg::FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    // one 32x32 block at a time, so that few addresses are live beside the sums; rows and
+    // k past the end read the last one and count as zero
+#pragma unroll
+    for (int fm = 0; fm < Cfg::FM; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < Cfg::FN; ++fn) {
+            const int r = m0 + fm * 32 + li, c = n0 + fn * 32 + li;
+            const float* pa = A + min(r, p.M - 1) * (TA ? 1 : p.lda);
+            const float* pb = B + min(c, p.N - 1) * (TB ? p.ldb : 1);
+            const long long da = TA ? p.lda : 1, db = TB ? 1 : p.ldb;
+#pragma unroll 1
+            for (int k0 = kBeg; k0 < kEnd; k0 += 16) {   // the lane halves take eight k each
+                float a[8], b[8];
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    const long long k = min(k0 + 8 * h + s, kEnd - 1);
+                    a[s] = pa[k * da];
+                    b[s] = pb[k * db];
+                }
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    const bool in = k0 + 8 * h + s < kEnd;
+                    acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && r < p.M ? a[s] : 0.f,
+                                                                       in && c < p.N ? b[s] : 0.f, acc[fm][fn], 0, 0, 0);
+                }
+            }
+        }
+}
 
+// 16-deep slices per LDS stage, and so per block barrier. The 64x64 tile has six
+// MFMAs per wave and slice: with one slice per barrier their time is less than the
+// fragment reads', the LDS stores' and the barrier's that every slice then waits for.
+template <class Cfg>
+constexpr int kSub = Cfg::FM * Cfg::FN == 1 ? 2 : 1;
+
+// LDS: two stages of both operands' pieces.
+template <class Cfg>
+constexpr int kSliceBytes = SplitLds<Cfg::BM>::SIZE + SplitLds<Cfg::BN>::SIZE;
+template <class Cfg>
+constexpr size_t ldsBytes() { return 2 * kSub<Cfg> * kSliceBytes<Cfg>; }
+
+// The main loop of one tile: stage T & 1 (SUB slices) is multiplied from LDS
+// while stage T + 1 goes from its registers to the other half of LDS and stage
+// T + 2 is loaded.
+template <class Cfg, bool TA, bool TB>
+__device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0,
+                                          int n0, long long batch, int kBeg, int kEnd, int wm, int wn, int lane,
+                                          int tid) {
+    constexpr int SUB = kSub<Cfg>, SLICE = kSliceBytes<Cfg>, STAGE = SUB * SLICE, OFF_B = SplitLds<Cfg::BM>::SIZE;
+    using LA = SplitLoader<!TA, Cfg::BM, Cfg::NT>;
+    using LB = SplitLoader<TB, Cfg::BN, Cfg::NT>;
+    LA la[SUB];
+    LB lb[SUB];
+    la[0].init(p.A + batch * p.sA, p.lda, p.M, m0, tid);
+    lb[0].init(p.B + batch * p.sB, p.ldb, p.N, n0, tid);
+#pragma unroll
+    for (int u = 1; u < SUB; ++u) {
+        la[u] = la[0];
+        lb[u] = lb[0];
+    }
+    const int nk = (kEnd - kBeg + 15) / 16, nFull = (kEnd - kBeg) / 16;
+    const int nt = (nk + SUB - 1) / SUB;   // stages; slices past nk are loaded as zeros
+    // FULL: stages T + 1 and T + 2 exist and are whole
+    auto step = [&](auto full, int T, int j) {
+        constexpr bool FULL = decltype(full)::value;
+        const char* cur = smem + j * STAGE;
+        char* oth = smem + (j ^ 1) * STAGE;
+        const bool st = FULL || T + 1 < nt, ld = FULL || T + 2 < nt;
+        auto side = [&](int u, int i) {
+            const int k0 = kBeg + ((T + 2) * SUB + u) * 16;
+            if (i < LA::PARTS) {
+                if (st) la[u].storePart(i, oth + u * SLICE, tid);
+                if (ld) la[u].template loadPart<FULL>(i, k0, kEnd, tid);
+            } else {
+                if (st) lb[u].storePart(i - LA::PARTS, oth + u * SLICE + OFF_B, tid);
+                if (ld) lb[u].template loadPart<FULL>(i - LA::PARTS, k0, kEnd, tid);
+            }
+        };
+        constexpr int SIDES = LA::PARTS + LB::PARTS;
+        if constexpr (SUB > 1)
+            mmaSplitSub<Cfg, SUB, SIDES, kSideValu>(cur, cur + OFF_B, SLICE, acc[0][0], wm, wn, lane, side);
+        else
+            mmaSplitSlice<Cfg, SIDES, kSideValu>(cur, cur + OFF_B, acc, wm, wn, lane, [&](int i) { side(0, i); });
+        __syncthreads();
+    };
+    // Stages 0 and 1 are loaded together (one memory latency before the first products, not
+    // two). The main loop's own first loads test nothing: its waits then count the same loads
+    // on every path (after a guarded load the compiler waits for all of them on each trip).
+    auto fill = [&](auto full) {
+        constexpr bool FULL = decltype(full)::value;
+        LA fa[SUB];
+        LB fb[SUB];
+#pragma unroll
+        for (int u = 0; u < SUB; ++u) {
+            fa[u] = la[0];
+            fb[u] = lb[0];
+            fa[u].template load<FULL>(kBeg + u * 16, kEnd, tid);
+            fb[u].template load<FULL>(kBeg + u * 16, kEnd, tid);
+        }
+        if (FULL || nt > 1) {
+#pragma unroll
+            for (int u = 0; u < SUB; ++u) {
+                la[u].template load<FULL>(kBeg + (SUB + u) * 16, kEnd, tid);
+                lb[u].template load<FULL>(kBeg + (SUB + u) * 16, kEnd, tid);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SUB; ++u) {
+            fa[u].store(smem + u * SLICE, tid);
+            fb[u].store(smem + u * SLICE + OFF_B, tid);
+        }
+        __syncthreads();
+    };
+    int T = 0;
+    if (nFull >= 4 * SUB) {
+        fill(std::true_type{});
+        for (; (T + 4) * SUB <= nFull; T += 2) {
+            step(std::true_type{}, T, 0);
+            step(std::true_type{}, T + 1, 1);
+        }
+    } else {
+        fill(std::false_type{});
+    }
+#pragma unroll 1
+    for (; T < nt; T += 2) {
+        step(std::false_type{}, T, 0);
+        if (T + 1 < nt) step(std::false_type{}, T + 1, 1);
+    }
+}
+
+// One output tile (bid: the tile's linear index, batch, split) of C =
+// op(A) * op(B). GATE: each element of C is kept where p.gate (same shape, row
+// stride p.ldg) is > 0 and set to 0 elsewhere (a ReLU's backward applied to the
+// product). PLAIN: on the fp32 MFMA from the start (strides beyond the buffer
+// views). Every tile adds a product's terms in the same order.
+template <class Cfg, bool TA, bool TB, bool PLAIN, bool GATE = false>
+__device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, int bid, long long batch, int split) {
+    static_assert(Cfg::BK == 16, "one MFMA step per slice");
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / Cfg::WAVES_N;
     const int wn = wave % Cfg::WAVES_N;
 
@@ -221,30 +279,6 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, float* smem,
     // This split's K range; the loaders treat kEnd as the end of K.
     const int kBeg = split * p.kChunk;
     const int kEnd = min(p.K, kBeg + p.kChunk);
-    // BSUM: thread tid < BN owns column n0 + tid; the slice at k0 is in the B
-    // region of an LDS stage as [BK][BN + 4].
-    const bool doSum = BSUM && p.colSum && tm == 0 && tid < Cfg::BN && n0 + tid < p.N;
-    float colAcc = 0.f;
-    // The slice's BK values are read first (all inside the LDS stage) and then added in
-    // row order; rows past the K range add -0.0f, which leaves every sum unchanged (a
-    // guarded read per row made each read wait alone: the first tile row's mainloop ran
-    // ~3x longer than the others').
-    auto colSum = [&](const float* sB, int k0) {
-        if constexpr (BSUM) {
-            if (doSum) {
-                float v[Cfg::BK];
-#pragma unroll
-                for (int k = 0; k < Cfg::BK; ++k) v[k] = sB[k * SB::LD + tid];
-#pragma unroll
-                for (int k = 0; k < Cfg::BK; ++k) colAcc += k0 + k < kEnd ? v[k] : -0.0f;
-            }
-        }
-    };
-
-    GemmLoader<A_KMAJOR, LA, Cfg::BM, Cfg::BK, Cfg::NT> la;
-    la.init(p.A + batch * p.sA, p.lda, p.M, m0, tid);
-    GemmLoader<B_KMAJOR, LB, Cfg::BN, Cfg::BK, Cfg::NT> lb;
-    lb.init(p.B + batch * p.sB, p.ldb, p.N, n0, tid);
 
     f32x16 acc[Cfg::FM][Cfg::FN];
 #pragma unroll
@@ -283,190 +317,66 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, float* smem,
             }
     }
 
-    const int nk = (kEnd - kBeg + Cfg::BK - 1) / Cfg::BK;
-    la.template load<false>(kBeg, kEnd, tid);
-    lb.template load<false>(kBeg, kEnd, tid);
-    la.store(smem, tid);
-    lb.store(smem + SA::SIZE, tid);
-    const int nFull = (kEnd - kBeg) / Cfg::BK;
-    int t = 0;
-    if constexpr (PRE) {
-        // Two slices in flight: while slice t is multiplied from LDS, slice t+1 (loaded
-        // one slice earlier) is stored to the other stage and slice t+2 is loaded into a
-        // second register set (la2 / lb2), so a load has two slices of MFMA work to land
-        // instead of one. The small tiles run one workgroup per CU with short main loops,
-        // where a single slice did not cover the load latency.
-        GemmLoader<A_KMAJOR, LA, Cfg::BM, Cfg::BK, Cfg::NT> la2;
-        la2.init(p.A + batch * p.sA, p.lda, p.M, m0, tid);
-        GemmLoader<B_KMAJOR, LB, Cfg::BN, Cfg::BK, Cfg::NT> lb2;
-        lb2.init(p.B + batch * p.sB, p.ldb, p.N, n0, tid);
-        if (nk > 1) {
-            la.template load<false>(kBeg + Cfg::BK, kEnd, tid);
-            lb.template load<false>(kBeg + Cfg::BK, kEnd, tid);
-        }
-        __syncthreads();
-        // Slice t is in stage t & 1; on entry to a trip la / lb hold slice t+1. The
-        // unchecked loop runs while the slices it fetches (t+2, t+3) are whole.
-        for (; t + 3 < nFull; t += 2) {
-            la2.template load<true>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-            lb2.template load<true>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-            __builtin_amdgcn_sched_barrier(0);
-            colSum(smem + SA::SIZE, kBeg + t * Cfg::BK);
-            mma_slice_split<Cfg, A_KMAJOR, B_KMAJOR>(smem, smem + SA::SIZE, acc, wm, wn, lane, [&] {
-                la.store(smem + STAGE, tid);
-                lb.store(smem + STAGE + SA::SIZE, tid);
-            });
-            __syncthreads();
-            la.template load<true>(kBeg + (t + 3) * Cfg::BK, kEnd, tid);
-            lb.template load<true>(kBeg + (t + 3) * Cfg::BK, kEnd, tid);
-            __builtin_amdgcn_sched_barrier(0);
-            colSum(smem + STAGE + SA::SIZE, kBeg + (t + 1) * Cfg::BK);
-            mma_slice_split<Cfg, A_KMAJOR, B_KMAJOR>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane, [&] {
-                la2.store(smem, tid);
-                lb2.store(smem + SA::SIZE, tid);
-            });
-            __syncthreads();
-        }
-        for (; t < nk; t += 2) {
-            if (t + 2 < nk) {
-                la2.template load<false>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-                lb2.template load<false>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-            }
-            colSum(smem + SA::SIZE, kBeg + t * Cfg::BK);
-            mma_slice<Cfg, A_KMAJOR, B_KMAJOR>(smem, smem + SA::SIZE, acc, wm, wn, lane);
-            if (t + 1 < nk) {
-                la.store(smem + STAGE, tid);
-                lb.store(smem + STAGE + SA::SIZE, tid);
-            }
-            __syncthreads();
-            if (t + 1 < nk) {
-                if (t + 3 < nk) {
-                    la.template load<false>(kBeg + (t + 3) * Cfg::BK, kEnd, tid);
-                    lb.template load<false>(kBeg + (t + 3) * Cfg::BK, kEnd, tid);
-                }
-                colSum(smem + STAGE + SA::SIZE, kBeg + (t + 1) * Cfg::BK);
-                mma_slice<Cfg, A_KMAJOR, B_KMAJOR>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
-                if (t + 2 < nk) {
-                    la2.store(smem, tid);
-                    lb2.store(smem + SA::SIZE, tid);
-                }
-                __syncthreads();
-            }
-        }
-    } else {
-        __syncthreads();
-        // Two slices per trip so both LDS stage addresses are compile-time
-        // offsets. The main loop runs while both slices it fetches (t+1, t+2) lie
-        // wholly inside the K range, so its loads test nothing; the last slices
-        // run in the checked loop below (slice t is always in stage t & 1). The
-        // schedule barriers keep each half in the order global loads, MFMAs, LDS
-        // stores, block barrier.
-        for (; t + 2 < nFull; t += 2) {
-            la.template load<true>(kBeg + (t + 1) * Cfg::BK, kEnd, tid);
-            lb.template load<true>(kBeg + (t + 1) * Cfg::BK, kEnd, tid);
-            __builtin_amdgcn_sched_barrier(0);
-            colSum(smem + SA::SIZE, kBeg + t * Cfg::BK);
-            mma_slice_split<Cfg, A_KMAJOR, B_KMAJOR>(smem, smem + SA::SIZE, acc, wm, wn, lane, [&] {
-                la.store(smem + STAGE, tid);
-                lb.store(smem + STAGE + SA::SIZE, tid);
-            });
-            __syncthreads();
-            la.template load<true>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-            lb.template load<true>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-            __builtin_amdgcn_sched_barrier(0);
-            colSum(smem + STAGE + SA::SIZE, kBeg + (t + 1) * Cfg::BK);
-            mma_slice_split<Cfg, A_KMAJOR, B_KMAJOR>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane, [&] {
-                la.store(smem, tid);
-                lb.store(smem + SA::SIZE, tid);
-            });
-            __syncthreads();
-        }
-        for (; t < nk; t += 2) {
-            {
-                const bool more = (t + 1) < nk;
-                if (more) {
-                    la.template load<false>(kBeg + (t + 1) * Cfg::BK, kEnd, tid);
-                    lb.template load<false>(kBeg + (t + 1) * Cfg::BK, kEnd, tid);
-                }
-                colSum(smem + SA::SIZE, kBeg + t * Cfg::BK);
-                mma_slice<Cfg, A_KMAJOR, B_KMAJOR>(smem, smem + SA::SIZE, acc, wm, wn, lane);
-                if (more) {
-                    la.store(smem + STAGE, tid);
-                    lb.store(smem + STAGE + SA::SIZE, tid);
-                }
-                __syncthreads();
-            }
-            if (t + 1 < nk) {
-                const bool more = (t + 2) < nk;
-                if (more) {
-                    la.template load<false>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-                    lb.template load<false>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
-                }
-                colSum(smem + STAGE + SA::SIZE, kBeg + (t + 1) * Cfg::BK);
-                mma_slice<Cfg, A_KMAJOR, B_KMAJOR>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
-                if (more) {
-                    la.store(smem, tid);
-                    lb.store(smem + SA::SIZE, tid);
-                }
-                __syncthreads();
-            }
-        }
+    bool plain = PLAIN;
+    if constexpr (!PLAIN) {
+        splitLoop<Cfg, TA, TB>(p, smem, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
+        plain = __any(unscaleSums(acc));
     }
+    if (plain)
+        plainProduct<Cfg, TA, TB>(p, acc, m0 + wm * Cfg::WM, n0 + wn * Cfg::WN, batch, kBeg, kEnd, lane);
 
     const int li = lane & 31, h = lane >> 5;
-    if constexpr (BSUM) {
-        if (doSum) p.colSum[n0 + tid] = colAcc;
-    }
-    if (p.ws) {
+    if constexpr (Cfg::BM * Cfg::BN <= 64 * 64) {   // the plans split K over the small tile only
         // Split-K: the last piece of the tile to arrive sums every piece's
         // partial product in split order and writes C.
-        if (!splitArrive<Cfg>(p, acc, smem, lane, batch, split, bid)) return;
+        if (p.ws && !splitArrive<Cfg>(p, acc, reinterpret_cast<float*>(smem), lane, batch, split, bid)) return;
     }
-    float* C = p.C + batch * p.sC;
-    const long long ldc = p.ldc;
+    // A lane's 16 rows of a block are 8 (r / 4) + r % 4 past its first one: a wave-uniform
+    // byte offset past its own. Rows and columns past the matrix get an offset out of the
+    // view's range and store nothing. (PLAIN: ldc may be beyond the view, 64-bit addresses.)
+    float* C = p.C + batch * p.sC + (long long)m0 * p.ldc + n0;
+    const auto rc = bufferRsrc(C, kSplitView);
     const bool bias = p.bias != nullptr;
     const bool relu = p.act == 1;
 #pragma unroll
     for (int fm = 0; fm < Cfg::FM; ++fm) {
+        const int rl = wm * Cfg::WM + fm * 32 + 4 * h;   // the lane's first row in the tile
 #pragma unroll
         for (int fn = 0; fn < Cfg::FN; ++fn) {
-            const int col = n0 + wn * Cfg::WN + fn * 32 + li;
-            if (col >= p.N) continue;
+            const int cl = wn * Cfg::WN + fn * 32 + li;
+            const bool colOk = n0 + cl < p.N;
             float b = 0.f;
             if constexpr (PRE) b = biasv[fn];
-            else b = bias ? p.bias[col] : 0.f;
+            else b = bias && colOk ? p.bias[n0 + cl] : 0.f;
+            const uint32_t voff = (uint32_t)((rl * p.ldc + cl) * 4);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm * Cfg::WM + fm * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                const int ro = 8 * (r >> 2) + (r & 3);
                 float v = acc[fm][fn][r];
                 if (bias) v += b;
                 if (relu) v = v > 0.f ? v : 0.f;
-                if (row < p.M) {
-                    if constexpr (GATE) v = gatev[fm][fn][r] > 0.f ? v : 0.f;
-                    C[(long long)row * ldc + col] = v;
+                if constexpr (GATE) v = gatev[fm][fn][r] > 0.f ? v : 0.f;
+                const bool in = colOk && m0 + rl + ro < p.M;
+                if constexpr (PLAIN) {
+                    if (in) C[(long long)(rl + ro) * p.ldc + cl] = v;
+                } else {
+                    bufStore1(rc, in ? voff : kSplitOOB, (uint32_t)(ro * p.ldc * 4), v);
                 }
             }
         }
     }
 }
 
-template <class Cfg, bool TA, bool TB, int LA, int LB>
-__global__ __launch_bounds__(Cfg::NT) void gemm_f32_kernel(GemmF32Params p) {
-    extern __shared__ float smem[];
-    gemmF32Tile<Cfg, TA, TB, LA, LB>(p, smem, blockIdx.x, blockIdx.z, blockIdx.y);
+template <class Cfg, bool TA, bool TB, bool PLAIN>
+__global__ __launch_bounds__(Cfg::NT, 2) void gemm_f32_kernel(GemmF32Params p) {
+    extern __shared__ __align__(16) char smem[];
+    gemmF32Tile<Cfg, TA, TB, PLAIN>(p, smem, blockIdx.x, blockIdx.z, blockIdx.y);
 }
 
-template <class Cfg, bool TA, bool TB>
-static size_t ldsBytesFor() {
-    using SA = LdsShape<!TA, Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<TB, Cfg::BN, Cfg::BK>;
-    return 2 * (SA::SIZE + SB::SIZE) * sizeof(float);
-}
-
-template <class Cfg, bool TA, bool TB, int LA, int LB>
+template <class Cfg, bool TA, bool TB, bool PLAIN>
 static int launchOne(const GemmF32Params& prm, int batch, int splits) {
-    auto kern = gemm_f32_kernel<Cfg, TA, TB, LA, LB>;
-    const size_t lds = ldsBytesFor<Cfg, TA, TB>();
+    auto kern = gemm_f32_kernel<Cfg, TA, TB, PLAIN>;
+    constexpr size_t lds = ldsBytes<Cfg>();
     OMHIP_CHECK(OMHIP_SET_MAX_DYNAMIC_LDS_ONCE(kern, lds));
     dim3 grid(prm.tilesM * prm.tilesN, splits, batch);
     hipLaunchKernelGGL(kern, grid, dim3(Cfg::NT), lds, stream(), prm);
@@ -474,38 +384,36 @@ static int launchOne(const GemmF32Params& prm, int batch, int splits) {
     return 0;
 }
 
-// In-tile byte offsets of the buffer-view loader stay below 2^30.
-template <bool KMAJOR, int R, int BK>
-static bool bufVecOk(bool vec, long long ld) {
-    const long long maxOff = KMAJOR ? ((long long)(R - 1) * ld + BK) * 4 : ((long long)(BK - 1) * ld + R) * 4;
-    return vec && maxOff < (long long)kMaxBufferBytes;
+// In-tile byte offsets of an operand's buffer view stay in range: R rows (at
+// most `rows` of them exist) of a 16-deep slice.
+static bool splitViewOk(bool kMajor, int R, int rows, long long ld) {
+    const long long maxOff = kMajor ? ((long long)(std::min(R, rows) - 1) * ld + 16) * 4 : (15 * ld + R) * 4;
+    return maxOff < (long long)kSplitView;
 }
 
-template <class Cfg, bool TA, bool TB>
-static int launchVec(GemmF32Params prm, int batch, int splits, bool va, bool vb) {
-    prm.tilesM = (prm.M + Cfg::BM - 1) / Cfg::BM;
-    prm.tilesN = (prm.N + Cfg::BN - 1) / Cfg::BN;
-    const bool ba = bufVecOk<!TA, Cfg::BM, Cfg::BK>(va, prm.lda);
-    const bool bb = bufVecOk<TB, Cfg::BN, Cfg::BK>(vb, prm.ldb);
-    if (ba && bb) return launchOne<Cfg, TA, TB, 2, 2>(prm, batch, splits);
-    if (va && vb) return launchOne<Cfg, TA, TB, 1, 1>(prm, batch, splits);
-    if (va) return launchOne<Cfg, TA, TB, 1, 0>(prm, batch, splits);
-    if (vb) return launchOne<Cfg, TA, TB, 0, 1>(prm, batch, splits);
-    return launchOne<Cfg, TA, TB, 0, 0>(prm, batch, splits);
-}
-
-// Slice depth of the large tile is a build-time constant (LDS: 2 x (256x(BK+4) + BKx260) floats).
 // The large tile runs 8 waves of 64 x 128 (two per SIMD, 128 accumulators
-// each): while one wave waits on its fragment reads, the block barrier or its
-// operand loads, the other keeps the SIMD's matrix core busy. On MI355X it
-// beats 4 waves of 128 x 128 (one per SIMD) by 5 % at 4096^3 and 8192^3 and
-// by 15 % at 8192 x 256 x 2048.
-#ifndef OMHIP_GEMM_BK
-#define OMHIP_GEMM_BK 16
-#endif
-using CfgL = TileCfg<256, 256, OMHIP_GEMM_BK, 64, 128>;
+// each): while one wave splits its share of the next slice or waits on its
+// fragment reads and the block barrier, the other keeps the matrix core busy.
+// It is bound by power: 4096^3 takes 570-605 us (227-241 TFLOP/s = 1.36-1.45
+// PFLOP/s of bf16 MFMA, what a library bf16 product of 8192^3 reaches on this
+// card, 1.37); on the fp32 MFMA it took 951-961 us (0.92 of that unit's peak).
+// Beside it: 8192^3 7.49 -> 4.74 ms, 3072^3 (128x128 tiles) 538 -> 345 us, 2048^3
+// 135 -> 100 us, 1001 x 765 x 1537 (TN, odd rows) 38.4 -> 29.7 us.
+using CfgL = TileCfg<256, 256, 16, 64, 128>;
 using CfgM = TileCfg<128, 128, 16, 64, 64>;
 using CfgS = TileCfg<64, 64, 16, 32, 32>;
+
+template <class Cfg, bool TA, bool TB>
+static int launchTile(GemmF32Params prm, int batch, int splits) {
+    prm.tilesM = (prm.M + Cfg::BM - 1) / Cfg::BM;
+    prm.tilesN = (prm.N + Cfg::BN - 1) / Cfg::BN;
+    if (splitViewOk(!TA, Cfg::BM, prm.M, prm.lda) && splitViewOk(TB, Cfg::BN, prm.N, prm.ldb) &&
+        splitViewOk(true, Cfg::BM, prm.M, prm.ldc + Cfg::BN))
+        return launchOne<Cfg, TA, TB, false>(prm, batch, splits);
+    prm.tilesM = (prm.M + CfgS::BM - 1) / CfgS::BM;
+    prm.tilesN = (prm.N + CfgS::BN - 1) / CfgS::BN;
+    return launchOne<CfgS, TA, TB, true>(prm, batch, splits);
+}
 
 // Tile and split-K choice (planGemmFor in gemm_f32.hpp) for this device.
 static GemmPlan planGemm(int M, int N, int K, int batch, bool wsOk) {
@@ -513,13 +421,11 @@ static GemmPlan planGemm(int M, int N, int K, int batch, bool wsOk) {
 }
 
 template <bool TA, bool TB>
-static int launchCfg(const GemmF32Params& prm, int batch, int splits, int cfg, bool va, bool vb) {
-    if (cfg == 0) return launchVec<CfgL, TA, TB>(prm, batch, splits, va, vb);
-    if (cfg == 1) return launchVec<CfgM, TA, TB>(prm, batch, splits, va, vb);
-    return launchVec<CfgS, TA, TB>(prm, batch, splits, va, vb);
+static int launchCfg(const GemmF32Params& prm, int batch, int splits, int cfg) {
+    if (cfg == 0) return launchTile<CfgL, TA, TB>(prm, batch, splits);
+    if (cfg == 1) return launchTile<CfgM, TA, TB>(prm, batch, splits);
+    return launchTile<CfgS, TA, TB>(prm, batch, splits);
 }
-
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Launches the GEMM (split-K: partials to ws, summed in the same launch by
 // each tile's last piece).
@@ -551,14 +457,11 @@ static int gemmF32Run(bool ta, bool tb, int batch, int M, int N, int K, const fl
             if (!prm.ctr) return -1;
         }
     }
-    // A is K-contiguous unless transposed; the vector axis is K (A) or M (A^T).
-    const bool va = aligned16(A) && lda % 4 == 0 && sA % 4 == 0 && (ta ? M % 4 == 0 : K % 4 == 0);
-    const bool vb = aligned16(B) && ldb % 4 == 0 && sB % 4 == 0 && (tb ? K % 4 == 0 : N % 4 == 0);
     int rc;
-    if (!ta && !tb) rc = launchCfg<false, false>(prm, batch, splits, plan.cfg, va, vb);
-    else if (!ta && tb) rc = launchCfg<false, true>(prm, batch, splits, plan.cfg, va, vb);
-    else if (ta && !tb) rc = launchCfg<true, false>(prm, batch, splits, plan.cfg, va, vb);
-    else rc = launchCfg<true, true>(prm, batch, splits, plan.cfg, va, vb);
+    if (!ta && !tb) rc = launchCfg<false, false>(prm, batch, splits, plan.cfg);
+    else if (!ta && tb) rc = launchCfg<false, true>(prm, batch, splits, plan.cfg);
+    else if (ta && !tb) rc = launchCfg<true, false>(prm, batch, splits, plan.cfg);
+    else rc = launchCfg<true, true>(prm, batch, splits, plan.cfg);
     return rc;
 }
 
@@ -607,27 +510,55 @@ int gemmF32Checked(const char* name, bool ta, bool tb, int batch, int M, int N, 
 }
 
 // ---- Linear backward in one launch -------------------------------------------
-// Workgroups [0, tilesW) compute dW = X^T G over 64 x 64 tiles, those of the
-// first tile row also adding G's columns into db (BSUM); the rest compute
-// dX = G W^T, kept where the gate is > 0 when one is given (GATE). K is not
-// split, so every element is the same sum, in the same order, as the separate
-// products compute whenever they do not split K either (e.g. every layer of the
-// 784-256-128-10 MLP at batch 128).
-template <int LK, bool GATE>
-__global__ __launch_bounds__(CfgS::NT) void linear_backward_kernel(GemmF32Params pw, GemmF32Params pa, int tilesW) {
-    extern __shared__ float smem[];
-    if ((int)blockIdx.x < tilesW)
-        gemmF32Tile<CfgS, true, false, LK, LK, true, false>(pw, smem, blockIdx.x, 0, 0);
-    else
-        gemmF32Tile<CfgS, false, true, LK, LK, false, GATE>(pa, smem, blockIdx.x - tilesW, 0, 0);
+// Workgroups [0, tilesW) compute dW = X^T G over 64 x 64 tiles, the next tilesX
+// dX = G W^T, kept where the gate is > 0 when one is given (GATE), and the last
+// ones G's column sums into db, a thread per column. K is not split, so every
+// element is the same sum, in the same order, as the separate products compute
+// whenever they do not split K either (e.g. every layer of the 784-256-128-10
+// MLP at batch 128).
+
+// colSum[col] = the sum of column col of G [rows, cols], row after row from 0.
+// Sixty-four rows are read at a time (each batch costs one memory latency: with
+// sixteen the sums of 128 rows outlasted the product tiles) and then added in row
+// order; rows past the end add -0.0f, which leaves every sum unchanged. The sums
+// have workgroups of their own: a product tile that also added its columns took
+// twice as long as its neighbours.
+__device__ __forceinline__ void columnSum(const float* G, float* colSum, int rows, int cols, int col) {
+    if (col >= cols) return;
+    float s = 0.f;
+    for (int k0 = 0; k0 < rows; k0 += 64) {
+        float v[64];
+#pragma unroll
+        for (int k = 0; k < 64; ++k) v[k] = G[(long long)min(k0 + k, rows - 1) * cols + col];
+#pragma unroll
+        for (int k = 0; k < 64; ++k) s += k0 + k < rows ? v[k] : -0.0f;
+    }
+    colSum[col] = s;
 }
 
-template <int LK, bool GATE>
-static int launchLinearBackward(const GemmF32Params& pw, const GemmF32Params& pa, int tilesW, int tilesX) {
-    auto kern = linear_backward_kernel<LK, GATE>;
-    const size_t lds = std::max(ldsBytesFor<CfgS, true, false>(), ldsBytesFor<CfgS, false, true>());
+constexpr int kSumCols = 64;   // columns per workgroup of the sums: many workgroups, one wave each
+
+template <bool PLAIN, bool GATE>
+__global__ __launch_bounds__(CfgS::NT) void linear_backward_kernel(GemmF32Params pw, GemmF32Params pa, int tilesW,
+                                                                  int tilesX, float* db) {
+    extern __shared__ __align__(16) char smem[];
+    const int b = blockIdx.x;
+    if (b < tilesW)
+        gemmF32Tile<CfgS, true, false, PLAIN>(pw, smem, b, 0, 0);
+    else if (b < tilesW + tilesX)
+        gemmF32Tile<CfgS, false, true, PLAIN, GATE>(pa, smem, b - tilesW, 0, 0);
+    else if (threadIdx.x < kSumCols)
+        columnSum(pw.B, db, pw.K, pw.N, (b - tilesW - tilesX) * kSumCols + threadIdx.x);
+}
+
+template <bool PLAIN, bool GATE>
+static int launchLinearBackward(const GemmF32Params& pw, const GemmF32Params& pa, int tilesW, int tilesX, float* db) {
+    auto kern = linear_backward_kernel<PLAIN, GATE>;
+    constexpr size_t lds = ldsBytes<CfgS>();
     OMHIP_CHECK(OMHIP_SET_MAX_DYNAMIC_LDS_ONCE(kern, lds));
-    hipLaunchKernelGGL(kern, dim3(tilesW + tilesX), dim3(CfgS::NT), lds, stream(), pw, pa, tilesW);
+    const int sums = db ? (pw.N + kSumCols - 1) / kSumCols : 0;
+    hipLaunchKernelGGL(kern, dim3(tilesW + tilesX + sums), dim3(CfgS::NT), lds, stream(), pw, pa,
+                       tilesW, tilesX, db);
     OMHIP_CHECK_LAUNCH();
     return 0;
 }
@@ -637,23 +568,23 @@ static int linearBackward(const float* X, const float* G, const float* W, const 
     GemmF32Params pw{}, pa{};
     // dW [I, O] = X^T G: A = X stored [K = B, M = I], B = G stored [K = B, N = O]
     pw.A = X; pw.B = G; pw.C = dW; pw.M = I; pw.N = O; pw.K = B;
-    pw.lda = I; pw.ldb = O; pw.ldc = O; pw.kChunk = B; pw.colSum = db;
+    pw.lda = I; pw.ldb = O; pw.ldc = O; pw.kChunk = B;
     pw.tilesM = (I + CfgS::BM - 1) / CfgS::BM; pw.tilesN = (O + CfgS::BN - 1) / CfgS::BN;
     // dX [B, I] = G W^T: A = G stored [M = B, K = O], B = W stored [N = I, K = O]
     pa.A = G; pa.B = W; pa.C = dX; pa.M = B; pa.N = I; pa.K = O;
     pa.lda = O; pa.ldb = O; pa.ldc = I; pa.kChunk = O; pa.gate = gate; pa.ldg = I;
     pa.tilesM = (B + CfgS::BM - 1) / CfgS::BM; pa.tilesN = (I + CfgS::BN - 1) / CfgS::BN;
     const long long tilesW = (long long)pw.tilesM * pw.tilesN, tilesX = dX ? (long long)pa.tilesM * pa.tilesN : 0;
-    if (tilesW + tilesX > 0x7fffffffLL) return fail("omHipLinearBackward: %lld tiles exceed the grid", tilesW + tilesX);
-    // 16-byte operand loads: every operand's contiguous axis (I or O) and base in whole vectors
-    bool vec = I % 4 == 0 && O % 4 == 0 && aligned16(X) && aligned16(G) && (!dX || aligned16(W));
-    vec = vec && bufVecOk<false, CfgS::BM, CfgS::BK>(true, I) && bufVecOk<false, CfgS::BN, CfgS::BK>(true, O) &&
-          bufVecOk<true, CfgS::BM, CfgS::BK>(true, O) && bufVecOk<true, CfgS::BN, CfgS::BK>(true, O);
-    if (vec)
-        return gate ? launchLinearBackward<2, true>(pw, pa, (int)tilesW, (int)tilesX)
-                    : launchLinearBackward<2, false>(pw, pa, (int)tilesW, (int)tilesX);
-    return gate ? launchLinearBackward<0, true>(pw, pa, (int)tilesW, (int)tilesX)
-                : launchLinearBackward<0, false>(pw, pa, (int)tilesW, (int)tilesX);
+    if (tilesW + tilesX + (O + kSumCols - 1) / kSumCols > 0x7fffffffLL) return fail("omHipLinearBackward: %lld tiles exceed the grid", tilesW + tilesX);
+    // X and G are walked along the batch, G and W along nOut
+    const bool views = splitViewOk(false, CfgS::BM, I, I) && splitViewOk(false, CfgS::BN, O, O) &&
+                       splitViewOk(true, CfgS::BM, B, O) && splitViewOk(true, CfgS::BN, I, O) &&
+                       splitViewOk(true, CfgS::BM, B, I + CfgS::BN);
+    if (views)
+        return gate ? launchLinearBackward<false, true>(pw, pa, (int)tilesW, (int)tilesX, db)
+                    : launchLinearBackward<false, false>(pw, pa, (int)tilesW, (int)tilesX, db);
+    return gate ? launchLinearBackward<true, true>(pw, pa, (int)tilesW, (int)tilesX, db)
+                : launchLinearBackward<true, false>(pw, pa, (int)tilesW, (int)tilesX, db);
 }
 
 // ---- fixed scratch of the no-allocation entry ---------------------------------

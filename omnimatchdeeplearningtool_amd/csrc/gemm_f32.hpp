@@ -11,35 +11,41 @@ struct GemmPlan {
     int splits;   // K splits (1: none)
 };
 
-// Tile and split-K choice on a device of `cus` compute units: the largest tile
-// that gives every CU a workgroup. When even 64x64 tiles give fewer than two
-// workgroups per CU and K is long (few rows or columns: 128 x 4096 x 4096,
-// weight gradients), K is split over the 64x64 tile: the smallest power of two
-// (at most 64) that gives every CU two workgroups while each split keeps >= 256
-// of K. The partials cost one fp32 write and read of C per split. Measured on
-// MI355X (TFLOP/s, against splitting the 128x128 tile until every CU had one
-// workgroup): 128 x 4096 x 4096 86 (76), 64 x 4096 x 4096 69 (56),
-// 128 x 1024 x 4096 47 (29), 512 x 1024 x 2048 72 (56), 256 x 4096 x 4096 96
-// (75). With 512 <= K < 1024 only grids of at most CUs / 4 tiles split (pieces
-// of >= 128 of K: 128 x 256 x 784, the MLP's first layer, 18.9 -> 11.5 us;
-// 256 x 512 x 768 18.9 -> 12.8; 512^3 14.2 -> 11.7); shorter K runs faster
-// unsplit. A split plan stops doubling once the grid holds 2 x CUs
-// workgroups, so its partials cover fewer than 4 x CUs tiles of 64 x 64
-// floats (16 MiB on 256 CUs). Host-only, so a CPU test checks that bound.
+// Tile and split-K choice on a device of `cus` compute units. A launch takes as
+// long as its busiest CU: tiles per CU times the time of one tile's 16-deep
+// slice, in us measured on MI355X (4096^3 forced onto each tile, divided by its
+// rounds; a lone small tile per CU from 1 x 1 rounds): 256x256 2.25, 128x128 0.66,
+// 64x64 0.23 (0.305 alone). Per 64x64 of C that is 0.141, 0.165, 0.23: the larger
+// tile splits each operand element for more products; the smaller one wins where
+// it fills the last round (4608^3: 324 tiles of 256x256 are two rounds, 4.5 against
+// 4.0 for 1296 of 128x128). Ties go to the larger tile.
+// When 64x64 tiles give fewer than two workgroups per CU and K is long (few rows
+// or columns: 128 x 4096 x 4096, weight gradients), K is split over the 64x64
+// tile: the smallest power of two (at most 64) that gives every CU two workgroups
+// while each split keeps >= 256 of K. The partials cost one fp32 write and read
+// of C per split. 128 x 4096 x 4096 measured (us): 1 split 78, 2 43, 4 38, 8 39.
+// With 512 <= K < 1024 only grids of at most CUs / 4 tiles split (pieces of >= 128
+// of K: 128 x 256 x 784, the MLP's first layer, 1 split 19.4, 2 13.4, 4 11.0,
+// 8 10.8); shorter K runs faster unsplit. A split plan stops doubling once the grid
+// holds 2 x CUs workgroups, so its partials cover fewer than 4 x CUs tiles of
+// 64 x 64 floats (16 MiB on 256 CUs). Host-only, so a CPU test checks that bound.
 inline GemmPlan planGemmFor(int M, int N, int K, int batch, bool wsOk, long long cus) {
     auto tiles = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-    if (tiles(256, 256) >= cus) return {0, 1};
-    if (tiles(128, 128) >= cus) return {1, 1};
     const long long t = tiles(64, 64);
+    auto rounds = [&](long long n) { return (double)((n + cus - 1) / cus); };
+    const double costL = 2.25 * rounds(tiles(256, 256)), costM = 0.66 * rounds(tiles(128, 128));
+    const double costS = t <= cus ? 0.305 : 0.23 * rounds(t);
+    if (costL <= costM && costL <= costS) return {0, 1};
+    if (costM <= costS) return {1, 1};
     if (t >= 2 * cus || !wsOk || K < 512 || (K < 1024 && t * 4 > cus)) return {2, 1};
     if (K < 1024) {   // very few tiles (at most CUs / 4): splits of >= 128 of K
         int s = 1;
         while (s < 64 && t * s < 2 * cus && K / (2 * s) >= 128) s *= 2;
         return {2, s};
     }
-    // with one tile per CU already, a split must keep >= 1024 of K (1024^3
-    // ran 79 TFLOP/s unsplit, 70 split in two)
-    const int minK = t >= cus ? 1024 : 256;
+    // with one tile per CU already, a split must keep >= 512 of K (1024^3: 24.5 us
+    // unsplit, 22.0 split in two)
+    const int minK = t >= cus ? 512 : 256;
     int s = 1;
     while (s < 64 && t * s < 2 * cus && K / (2 * s) >= minK) s *= 2;
     return {2, s};
@@ -78,7 +84,6 @@ struct GemmF32Params {
     int act;                // 0 identity, 1 ReLU (after the bias)
     const float* gate;      // Linear backward: C kept where gate > 0 (row stride ldg)
     long long ldg;
-    float* colSum;          // Linear backward: B's column sums (the bias gradient)
 };
 
 // C[b] = op(A[b]) * op(B[b]); ta: A stored [K,M]; tb: B stored [N,K].

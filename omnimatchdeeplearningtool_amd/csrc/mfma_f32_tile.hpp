@@ -52,83 +52,6 @@ struct LdsShape {
 };
 
 // ---------------------------------------------------------------------------
-// Dense operand loader: element (r,k) of a row-major matrix, KMAJOR or RMAJOR.
-// VEC loads 4 consecutive floats along the contiguous axis; the host enables it
-// only when that axis length, the leading dimension and the base are multiples
-// of 4 floats, so a vector is either fully inside the matrix or fully outside.
-// ---------------------------------------------------------------------------
-template <bool KMAJOR, bool VEC, int R, int BK, int NT>
-struct DenseLoader {
-    static constexpr int ELEMS = R * BK;
-    static constexpr int PER_T = VEC ? ELEMS / 4 / NT : ELEMS / NT;
-    static_assert(ELEMS % (NT * (VEC ? 4 : 1)) == 0, "tile must split evenly over threads");
-    using Shape = LdsShape<KMAJOR, R, BK>;
-
-    const float* p;   // operand base (this batch)
-    long long ld;
-    int rows;         // valid extent along r
-    int K;
-    int r0;           // tile origin along r
-    f32x4 v4[VEC ? PER_T : 1];
-    float v1[VEC ? 1 : PER_T];
-
-    __device__ void load(int k0, int tid) {
-        if constexpr (VEC) {
-#pragma unroll
-            for (int i = 0; i < PER_T; ++i) {
-                const int e = tid + i * NT;
-                int r, k;
-                if constexpr (KMAJOR) { r = e / (BK / 4); k = (e % (BK / 4)) * 4; }
-                else { k = e / (R / 4); r = (e % (R / 4)) * 4; }
-                const int gr = r0 + r, gk = k0 + k;
-                f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                if (gr < rows && gk < K) {
-                    const float* src = KMAJOR ? p + (long long)gr * ld + gk : p + (long long)gk * ld + gr;
-                    v = *reinterpret_cast<const f32x4*>(src);
-                }
-                v4[i] = v;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < PER_T; ++i) {
-                const int e = tid + i * NT;
-                int r, k;
-                if constexpr (KMAJOR) { r = e / BK; k = e % BK; }
-                else { k = e / R; r = e % R; }
-                const int gr = r0 + r, gk = k0 + k;
-                float v = 0.f;
-                if (gr < rows && gk < K)
-                    v = KMAJOR ? p[(long long)gr * ld + gk] : p[(long long)gk * ld + gr];
-                v1[i] = v;
-            }
-        }
-    }
-
-    __device__ void store(float* s, int tid) const {
-        if constexpr (VEC) {
-#pragma unroll
-            for (int i = 0; i < PER_T; ++i) {
-                const int e = tid + i * NT;
-                int r, k;
-                if constexpr (KMAJOR) { r = e / (BK / 4); k = (e % (BK / 4)) * 4; }
-                else { k = e / (R / 4); r = (e % (R / 4)) * 4; }
-                float* dst = KMAJOR ? s + r * Shape::LD + k : s + k * Shape::LD + r;
-                *reinterpret_cast<f32x4*>(dst) = v4[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < PER_T; ++i) {
-                const int e = tid + i * NT;
-                int r, k;
-                if constexpr (KMAJOR) { r = e / BK; k = e % BK; }
-                else { k = e / R; r = e % R; }
-                s[KMAJOR ? r * Shape::LD + k : k * Shape::LD + r] = v1[i];
-            }
-        }
-    }
-};
-
-// ---------------------------------------------------------------------------
 // Fragment reads + MFMA over one LDS slice.
 // ---------------------------------------------------------------------------
 template <class Cfg, bool A_KMAJOR, bool B_KMAJOR>
@@ -173,73 +96,6 @@ __device__ __forceinline__ void mma_slice(const float* __restrict__ sA, const fl
                 for (int fn = 0; fn < Cfg::FN; ++fn)
                     acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[fm][s], b[fn][s], acc[fm][fn], 0, 0, 0);
     }
-}
-
-// The MFMAs of one LDS slice with `mid` run between its first and second
-// halves: every fragment of the slice is read first, then the first half of
-// the k steps, mid() (the next slice's LDS stores), the second half. The
-// schedule barriers keep that order, so the stores' LDS traffic overlaps the
-// second half's MFMAs instead of sitting between the last MFMA and the block
-// barrier.
-template <class Cfg, bool A_KMAJOR, bool B_KMAJOR, class Mid>
-__device__ __forceinline__ void mma_slice_split(const float* __restrict__ sA, const float* __restrict__ sB,
-                                                f32x16 (&acc)[Cfg::FM][Cfg::FN], int wm, int wn, int lane,
-                                                Mid&& mid) {
-    using SA = LdsShape<A_KMAJOR, Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<B_KMAJOR, Cfg::BN, Cfg::BK>;
-    constexpr int U = Cfg::KH / 4;
-    static_assert(U % 2 == 0, "two halves of k steps");
-    const int li = lane & 31;
-    const int h = lane >> 5;
-    const int kb = h * Cfg::KH;
-    float a[U][Cfg::FM][4], b[U][Cfg::FN][4];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int fm = 0; fm < Cfg::FM; ++fm) {
-            const int row = wm * Cfg::WM + fm * 32 + li;
-            if constexpr (A_KMAJOR) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(sA + row * SA::LD + kb + 4 * u);
-                a[u][fm][0] = v[0]; a[u][fm][1] = v[1]; a[u][fm][2] = v[2]; a[u][fm][3] = v[3];
-            } else {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) a[u][fm][s] = sA[(kb + 4 * u + s) * SA::LD + row];
-            }
-        }
-#pragma unroll
-        for (int fn = 0; fn < Cfg::FN; ++fn) {
-            const int col = wn * Cfg::WN + fn * 32 + li;
-            if constexpr (B_KMAJOR) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(sB + col * SB::LD + kb + 4 * u);
-                b[u][fn][0] = v[0]; b[u][fn][1] = v[1]; b[u][fn][2] = v[2]; b[u][fn][3] = v[3];
-            } else {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) b[u][fn][s] = sB[(kb + 4 * u + s) * SB::LD + col];
-            }
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < U / 2; ++u)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int fm = 0; fm < Cfg::FM; ++fm)
-#pragma unroll
-                for (int fn = 0; fn < Cfg::FN; ++fn)
-                    acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][fm][s], b[u][fn][s], acc[fm][fn], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    mid();
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = U / 2; u < U; ++u)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int fm = 0; fm < Cfg::FM; ++fm)
-#pragma unroll
-                for (int fn = 0; fn < Cfg::FN; ++fn)
-                    acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][fm][s], b[u][fn][s], acc[fm][fn], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
 }
 
 // ---------------------------------------------------------------------------

@@ -1,0 +1,117 @@
+"""fp32 GEMM through bf16 pieces: every tile at its edges, and the values that the pieces carry with
+difficulty (denormals) or not at all (infinities, NaN, huge values), against float64.
+
+Bound: each output is a sum of K products; in any order, with every product and addition rounded to
+fp32 and (6 of 9 piece products) at most 2^-24 of each product left out, it is within
+(K + 2) 2^-24 sum |a b| of the exact sum, plus the smallest denormal for each of those roundings (tiles
+recomputed on the fp32 MFMA round every addition to the denormal spacing).
+"""
+import numpy as np
+import pytest
+
+from conftest import empty_dev, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# (M, N): 64x64 tiles, 128x128 tiles (one per CU / several), 256x256 tiles on a 256-CU device, each also ragged
+TILES = [(64, 64), (65, 131), (2048, 2048), (1930, 2047), (2048, 4096), (2047, 3970), (4096, 4096), (4090, 3845)]
+DEPTHS = [1, 15, 16, 17, 33, 64, 80, 81, 97, 112, 129]   # 1 .. 9 slices of 16, whole and partial
+
+
+def _operands(M, N, K, seed):
+    r = np.random.default_rng(seed)
+    return r.standard_normal((M, K), dtype=np.float32), r.standard_normal((K, N), dtype=np.float32)
+
+
+def _run(hip, layout, A, B):
+    M, K = A.shape
+    N = B.shape[1]
+    dC = empty_dev(hip, (M, N))
+    H = hip.HIPBackend
+    if layout == "nn":
+        H.matmul(to_dev(hip, A), to_dev(hip, B), dC, M, K, N)
+    elif layout == "nt":
+        H.matmulTransB(to_dev(hip, A), to_dev(hip, B.T), dC, M, K, N)
+    elif layout == "tn":
+        H.matmulTransA(to_dev(hip, A.T), to_dev(hip, B), dC, M, K, N)
+    else:
+        H.gemmStridedBatched(True, True, 1, M, N, K, to_dev(hip, A.T), M, 0, to_dev(hip, B.T), K, 0, dC, N, 0)
+    return dC.numpy()
+
+
+def _check(got, A, B, rows):
+    a, b = A[rows].astype(np.float64), B.astype(np.float64)
+    with np.errstate(all="ignore"):
+        ref = a @ b
+        mag = np.abs(a) @ np.abs(b)
+    got = got[rows].astype(np.float64)
+    fine = np.isfinite(ref) & (mag < 3.0e38)
+    over = ~np.isfinite(ref)
+    assert np.array_equal(np.isnan(got[over]), np.isnan(ref[over]))
+    inf = over & np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf])
+    bound = (A.shape[1] + 2) * (2.0 ** -24 * mag + 2.0 ** -149)
+    assert np.all(np.abs(got[fine] - ref[fine]) <= bound[fine])
+    return fine
+
+
+def _rows(M):
+    """All rows of a small product, else the edges of the tiles and some between."""
+    if M <= 160:
+        return np.arange(M)
+    return np.unique(np.r_[0:3, 62:66, 126:130, 254:258, np.arange(300, M, 211), M - 70:M - 60, M - 3:M])
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N", TILES)
+def test_tile_edges(hip, layout, M, N):
+    for K in DEPTHS if M * N < 1 << 16 else DEPTHS[1::3]:
+        print(f"case {layout} {M}x{N}x{K}", flush=True)
+        A, B = _operands(M, N, K, M + N + K)
+        assert _check(_run(hip, layout, A, B), A, B, _rows(M)).all()
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N,K", [(70, 67, 40), (128, 256, 2048), (2048, 2048, 50), (2048, 4096, 50), (4096, 4096, 50)])
+def test_special_values(hip, layout, M, N, K):
+    """Infinities, NaN, huge values and denormals in single elements; 128x256x2048 splits K."""
+    A, B = _operands(M, N, K, 7)
+    A[3, 5], A[9, 0], A[M - 1, K - 1] = np.inf, np.nan, -np.inf
+    A[12, :] = 0
+    A[12, 7] = np.inf                       # inf * b, and 0 elsewhere
+    A[20, 4], B[4, 11] = 3.3e38, 1e-30      # beyond the pieces' range, finite products
+    A[21, 6] = -2.7e33                      # 2^111 and above
+    B[6, :] *= np.float32(1e-20)
+    A[30, :] = np.float32(1e-42)            # denormal
+    A[31, :] = np.float32(3e-39)
+    A[32, :] *= np.float32(1e-36)
+    B[:, 20] *= np.float32(1e-38)
+    print(f"case {layout} {M}x{N}x{K}", flush=True)
+    _check(_run(hip, layout, A, B), A, B, np.unique(np.r_[0:40, M - 2:M]))
+
+
+@pytest.mark.parametrize("scale_a,scale_b", [(1e-42, 1e36), (1e-40, 1e-2), (1e-37, 1e-5), (1e32, 1e-32), (1e18, 1e19)])
+def test_ranges(hip, scale_a, scale_b):
+    """Whole operands of denormals, tiny and huge values (the last two near and past the pieces' range)."""
+    A, B = _operands(130, 70, 45, 3)
+    A, B = A * np.float32(scale_a), B * np.float32(scale_b)
+    _check(_run(hip, "nn", A, B), A, B, np.arange(130))
+
+
+def test_linear_backward_special_values(hip):
+    """The fused backward's products and column sums with a huge and an infinite gradient element."""
+    H = hip.HIPBackend
+    nb, ni, no = 37, 70, 66
+    r = np.random.default_rng(5)
+    X, G, W = (r.standard_normal(s, dtype=np.float32) for s in ((nb, ni), (nb, no), (ni, no)))
+    X[4, :] = 0
+    G[4, 9], G[7, 20], G[8, 21] = 3e38, np.inf, 1e-42
+    dW, db, dX = empty_dev(hip, (ni, no)), empty_dev(hip, (no,)), empty_dev(hip, (nb, ni))
+    H.linearBackward(to_dev(hip, X), to_dev(hip, G), to_dev(hip, W), None, dW, db, dX, nb, ni, no)
+    want = np.zeros(no, np.float32)
+    for row in G:
+        want = want + row
+    assert np.array_equal(db.numpy(), want)
+    _check(dW.numpy(), np.ascontiguousarray(X.T), G, np.arange(ni))
+    keep = np.setdiff1d(np.arange(nb), [4])   # row 4 overflows
+    _check(dX.numpy(), G, np.ascontiguousarray(W.T), keep)
