@@ -28,13 +28,14 @@ DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON = ["-O3", "-std=c++20", "-fPIC", "-Wall", "-Wno-unused-function", "-Wno-unused-variable"]
 
 SOURCES = ["runtime.cpp", "eltwise.hip", "gemm_f32.hip", "conv.hip", "conv_stem.hip", "conv_wgrad.hip", "gemm_half.hip", "gemm_half_heads.hip", "train.hip",
-           "pool.hip", "attention.hip", "infer.hip", "loss.hip", "mha.hip", "heads.hip"]
+           "pool.hip", "attention.hip", "attention_f32.hip", "infer.hip", "loss.hip", "mha.hip", "heads.hip"]
 # conv tiles keep at most 128 accumulators per lane: forcing the VGPR form of
 # the MFMA operands stops the register allocator from copying every
 # accumulator between AGPRs and VGPRs on each trip of the mainloop (and, in
 # the fused attention, every score back to VGPRs for the softmax).
 EXTRA_FLAGS = {"conv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "conv_stem.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "conv_wgrad.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-               "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+               "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+               "attention_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd):
