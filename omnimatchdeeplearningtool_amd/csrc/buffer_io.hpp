@@ -55,4 +55,12 @@ __device__ __forceinline__ float bufLoad1Agent(__amdgpu_buffer_rsrc_t r, uint32_
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kCpolAgent));
 }
 
+__device__ __forceinline__ void bufStore4Agent(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, f32x4 v) {
+    typedef uint32_t u32x4b __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4b, v), r, voff, soff, kCpolAgent);
+}
+__device__ __forceinline__ f32x4 bufLoad4Agent(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kCpolAgent));
+}
+
 }  // namespace omhip
