@@ -203,9 +203,10 @@ int omHipMergeHeads(const float* pIn, float* pOut, int nBatch, int nSeqLen, int 
  * (vit.ixx:163-187): qkvSplitHeads (Q times fScale), tensorTranspose2dBatched +
  * tensorBatchedMatmul (Q K^T), tensorSoftmaxLastDim, tensorBatchedMatmul (P V),
  * mergeHeads. pQKV [nBatch*nSeq, 3*D] -> pOut [nBatch*nSeq, D], both fp32. Q is scaled as
- * qkvSplitHeads scales it; the products read the heads where they lie (no transpose or split
- * copy) and accumulate in fp32; the softmax is omHipSoftmax's. Intermediates use the
- * stream's staging workspace. */
+ * qkvSplitHeads scales it and products accumulate in fp32. Head dimensions that are multiples
+ * of 4 up to 128 run as one kernel without intermediates (running maximum over the keys);
+ * others as strided products that read the heads where they lie and omHipSoftmax, with
+ * intermediates in the stream's staging workspace. */
 int omHipAttention(const float* pQKV, float* pOut, int nBatch, int nSeq, int nHeads, int nHeadDim, float fScale);
 
 /* ===== fp32 GEMM (cuda_kernels.cuh:109-117) ===== */
