@@ -198,6 +198,9 @@ int launchAttnF32(const AttnF32Params& p, int blocks) {
 
 bool attentionF32Fits(int B, int S, int H, int hd) {
     const long long blocks = (long long)B * H * ((S + kQueries - 1) / kQueries);
+    // A workgroup walks all keys of its head alone (about 3 us per 64): beyond 512 keys that pays only where
+    // every CU has a workgroup; the composed path's products spread a few long heads over the card.
+    if (S > 512 && blocks < cuCount()) return false;
     // 16-byte loads of four d; a tile's rows in one buffer view
     return hd % 4 == 0 && hd <= kAttnF32MaxHeadDim && blocks <= 0x7fffffffLL &&
            3LL * H * hd * 4 * kKeys <= (long long)kMaxBufferBytes;
