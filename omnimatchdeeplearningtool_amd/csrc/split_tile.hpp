@@ -164,6 +164,7 @@ struct SplitLoaderR {
     template <bool FULL>
     __device__ __forceinline__ void loadPart(int i, int k0, int kEnd, int tid) {
         const auto rs = bufferRsrc(tile + (long long)k0 * ld, kSplitView);
+        // the k rows' offset is the scalar one: added to a marked row's kSplitOOB it would wrap into range
         const uint32_t step = (uint32_t)ld * 4u;
         if (FULL || k0 + Lds::BK <= kEnd) {
 #pragma unroll
@@ -171,7 +172,7 @@ struct SplitLoaderR {
         } else {
             const int k = k0 + tid / R * KU;
 #pragma unroll
-            for (int j = 4 * i; j < 4 * i + 4; ++j) v[j] = bufLoad1(rs, k + j < kEnd ? voff + j * step : kSplitOOB, 0);
+            for (int j = 4 * i; j < 4 * i + 4; ++j) v[j] = bufLoad1(rs, k + j < kEnd ? voff : kSplitOOB, j * step);
         }
     }
 

@@ -90,6 +90,31 @@ def test_special_values(hip, layout, M, N, K):
     _check(_run(hip, layout, A, B), A, B, np.unique(np.r_[0:40, M - 2:M]))
 
 
+@pytest.mark.parametrize("M,N", [(50, 45), (70, 67), (13, 131)])
+@pytest.mark.parametrize("ta,tb", [(True, False), (False, False), (True, True)])
+def test_row_padding_is_not_read(hip, ta, tb, M, N):
+    """Rows of an operand stored K first are longer than the matrix: what lies behind them (NaN here) is read
+    neither by whole slices nor by the last, partial one, so the sums are the same bits as with zeros there (a NaN
+    in any lane's sums would send its block to the fp32 MFMA, which rounds differently)."""
+    pad = 96
+    for K in (7, 45, 128, 141):
+        print(f"case {ta} {tb} {M}x{N}x{K}", flush=True)
+        A, B = _operands(M, N, K, K)
+        got = []
+        for fill in (0.0, np.nan):
+            a, b = (np.ascontiguousarray(x) for x in (A.T if ta else A, B.T if tb else B))
+            lda, ldb = a.shape[1], b.shape[1]
+            if ta:
+                a, lda = np.c_[a, np.full((K, pad), fill, np.float32)], M + pad
+            if not tb:
+                b, ldb = np.c_[b, np.full((K, pad), fill, np.float32)], N + pad
+            dC = empty_dev(hip, (M, N))
+            hip.HIPBackend.gemmStridedBatched(ta, tb, 1, M, N, K, to_dev(hip, a), lda, 0, to_dev(hip, b), ldb, 0, dC, N, 0)
+            got.append(dC.numpy())
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+        assert _check(got[0], A, B, np.arange(M)).all()
+
+
 @pytest.mark.parametrize("scale_a,scale_b", [(1e-42, 1e36), (1e-40, 1e-2), (1e-37, 1e-5), (1e32, 1e-32), (1e18, 1e19)])
 def test_ranges(hip, scale_a, scale_b):
     """Whole operands of denormals, tiny and huge values (the last two near and past the pieces' range)."""
