@@ -341,6 +341,7 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
 #pragma unroll
     for (int fm = 0; fm < Cfg::FM; ++fm) {
         const int rl = wm * Cfg::WM + fm * 32 + 4 * h;   // the lane's first row in the tile
+        const int rowsLeft = p.M - m0 - wm * Cfg::WM - fm * 32;
 #pragma unroll
         for (int fn = 0; fn < Cfg::FN; ++fn) {
             const int cl = wn * Cfg::WN + fn * 32 + li;
@@ -360,7 +361,7 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
                 if constexpr (PLAIN) {
                     if (in) C[(long long)(rl + ro) * p.ldc + cl] = v;
                 } else {
-                    bufStore1(rc, in ? voff : kSplitOOB, (uint32_t)(ro * p.ldc * 4), v);
+                    bufStore1(rc, in ? voff : kSplitOOB, storeRowOffset(ro, rowsLeft, p.ldc), v);
                 }
             }
         }

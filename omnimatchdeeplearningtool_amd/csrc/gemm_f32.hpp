@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstddef>
+#include <cstdint>
 
 namespace omhip {
 
@@ -67,6 +68,19 @@ inline int splitPieces(int K, int splits, int* kChunk = nullptr) {
 // zero); the partials use the rest.
 constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
 constexpr size_t kNoAllocCounterBytes = (size_t)64 << 10;
+
+// The buffer views of the operands and of C reach almost 2^32 bytes past their
+// first element; a lane whose offset is kSplitOOB reads zero and writes nothing
+// beside any scalar offset that lies inside the view (the range check is
+// kSplitOOB >= kSplitView - scalar offset).
+constexpr uint32_t kSplitView = 0xffffff00u, kSplitOOB = 0xffffff80u;
+
+// Scalar byte offset of the C rows `ro` past a wave block's first, of which
+// `rowsLeft` exist: 0 for rows that no lane writes, whose own offset could be any
+// value mod 2^32 (a matrix of few rows may have a row stride of 2^30).
+constexpr uint32_t storeRowOffset(int ro, int rowsLeft, long long ldc) {
+    return ro < rowsLeft ? (uint32_t)(ro * ldc * 4) : 0u;
+}
 
 struct GemmF32Params {
     const float* A;

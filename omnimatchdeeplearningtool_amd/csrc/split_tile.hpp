@@ -30,6 +30,7 @@
 #include <cstdint>
 
 #include "buffer_io.hpp"
+#include "gemm_f32.hpp"
 #include "mfma_f32_tile.hpp"
 
 namespace omhip {
@@ -69,10 +70,6 @@ struct SplitLds {
     static constexpr int PIECE = 2 * GROUP;
     static constexpr int SIZE = 3 * PIECE;   // bytes
 };
-
-// The loaders' buffer views reach almost 2^32 bytes past a slice's first element;
-// a lane whose offset is kSplitOOB reads zero.
-constexpr uint32_t kSplitView = 0xffffff00u, kSplitOOB = 0xffffff80u;
 
 // Loader of a K-contiguous operand: element (r, k) at P[r * ld + k], in
 // 4-float vectors (any 4-byte alignment). Per-lane byte offsets are fixed for

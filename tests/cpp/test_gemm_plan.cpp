@@ -3,8 +3,11 @@
 // (kNoAllocScratchBytes less its arrival counters), the tiles' counters fit
 // theirs (kNoAllocCounterBytes), and the partials stay below the stated bound of 4 x CUs tiles of
 // 64 x 64 floats, over the GEMM sweep, the MLP and ResNet weight-gradient
-// shapes, the shapes that reach the bound, and a dense grid of small M / N.
+// shapes, the shapes that reach the bound, and a dense grid of small M / N. And of
+// the C store's offsets: whatever the row stride, a row past the matrix stays out of
+// the buffer view and a row inside it keeps its offset.
 // Exit status 0 = all checks passed.
+#include <cstdint>
 #include <cstdio>
 #include <vector>
 
@@ -31,7 +34,31 @@ static void check(int M, int N, int K, int batch, long long cus) {
     }
 }
 
+// Range check of a raw buffer access: the lane's offset against the view's bytes less the scalar offset, all 32 bits.
+static bool outOfRange(uint32_t lane, uint32_t scalar) { return lane >= (uint32_t)(omhip::kSplitView - scalar); }
+
+static void checkStore(int M, long long ldc) {
+    // the host takes the buffer views only while a 64-row tile's existing rows lie inside one
+    if (((M < 64 ? M : 64) - 1) * ldc * 4 + 512 >= (long long)omhip::kSplitView) return;
+    for (int block = 0; block < 64; block += 32)
+        for (int r = 0; r < 16; ++r) {
+            const int ro = 8 * (r >> 2) + (r & 3), left = M - block;
+            const uint32_t off = omhip::storeRowOffset(ro, left, ldc);
+            if (!outOfRange(omhip::kSplitOOB, off) || (ro < left && off != (uint64_t)ro * ldc * 4)) {
+                std::printf("FAIL store M=%d ldc=%lld block %d row %d: offset %u\n", M, ldc, block, ro, off);
+                ++g_fail;
+            }
+        }
+}
+
 int main() {
+    for (int M : {1, 2, 3, 9, 17, 28, 31, 33, 60, 64, 200}) {
+        for (long long ldc : {1LL, 64LL, 4096LL, 1LL << 24, (1LL << 30) - 1, 1LL << 30}) checkStore(M, ldc);
+        // strides whose multiples fall just past the view's end, mod 2^32
+        for (int ro = 1; ro < 28; ++ro)
+            for (uint64_t at = 0xfffffe80u; at < 0x100000080u; at += 4)
+                for (uint64_t w = 0; w < 4; ++w) checkStore(M, (long long)((at + (w << 32)) / 4 / ro));
+    }
     const int sq[] = {512, 1024, 2048, 4096, 8192};
     for (int s : sq) check(s, s, s, 1, 256);
     check(128, 4096, 4096, 1, 256);
