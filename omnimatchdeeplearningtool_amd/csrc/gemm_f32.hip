@@ -90,10 +90,10 @@ __device__ __forceinline__ bool splitArrive(const GemmF32Params& p, f32x16 (&acc
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int i = 0; i < Cfg::FM * Cfg::FN * 4; ++i)   // splits past the last read zero (out of range)
+            for (int i = 0; i < Cfg::FM * Cfg::FN * 4; ++i)   // splits past the last are out of range: zero, no access
                 w[j][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                    rw, s0 + j < p.splits ? laneOff + (uint32_t)i * 1024u : kOOB, base + (uint32_t)(s0 + j) * stride,
-                    kCpolAgent));
+                    rw, s0 + j < p.splits ? laneOff + (uint32_t)i * 1024u : kOOB,
+                    splitPartOffset(s0 + j, p.splits, base, stride), kCpolAgent));
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (s0 + j >= p.splits) break;

@@ -82,6 +82,13 @@ constexpr uint32_t storeRowOffset(int ro, int rowsLeft, long long ldc) {
     return ro < rowsLeft ? (uint32_t)(ro * ldc * 4) : 0u;
 }
 
+// Scalar byte offset of a tile's part `s` of `splits` among the split-K partials:
+// 0 for parts past the last, whose lanes are marked out of range (their own offset
+// lies past the view, where the range check's difference would wrap).
+constexpr uint32_t splitPartOffset(int s, int splits, uint32_t base, uint32_t stride) {
+    return s < splits ? base + (uint32_t)s * stride : 0u;
+}
+
 struct GemmF32Params {
     const float* A;
     const float* B;
@@ -91,7 +98,7 @@ struct GemmF32Params {
     long long sA, sB, sC;   // per-batch element offsets (0 shares the operand)
     int tilesM, tilesN;
     int kChunk;             // split-K: split s covers k in [s*kChunk, min(K, (s+1)*kChunk))
-    float* ws;              // split-K partials [split][batch][M][N] (null: write C directly)
+    float* ws;              // split-K partials [split][batch][tile], each tile in its registers' order (null: write C)
     unsigned* ctr;          // split-K: per (batch, tile) arrival counters, zero at rest
     int splits;             // split-K: pieces of K (the last arrival of a tile sums them)
     const float* bias;      // [N] added to every row of C, or null

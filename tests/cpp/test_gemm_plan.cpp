@@ -51,7 +51,24 @@ static void checkStore(int M, long long ldc) {
         }
 }
 
+// Every read of the partials: four parts at a time, those past the last out of range.
+static void checkParts(int splits, uint32_t tiles) {
+    const uint32_t view = tiles * splits * 64 * 64 * 4, stride = tiles * 64 * 64 * 4;
+    for (uint32_t slot : {0u, tiles - 1})
+        for (int s = 0; s < (splits + 3) / 4 * 4; ++s) {
+            const uint32_t off = omhip::splitPartOffset(s, splits, slot * 64 * 64 * 4, stride);
+            const uint32_t lane = s < splits ? 64 * 64 * 4 - 16 : 0x40000000u;   // kOOB
+            const bool out = lane >= (uint32_t)(view - off);
+            if (out == (s < splits) || (s < splits && (uint64_t)lane + off + 16 > view)) {
+                std::printf("FAIL parts splits=%d tiles=%u slot %u part %d: offset %u\n", splits, tiles, slot, s, off);
+                ++g_fail;
+            }
+        }
+}
+
 int main() {
+    for (int splits = 2; splits <= 64; ++splits)
+        for (uint32_t tiles : {1u, 3u, 64u, 511u}) checkParts(splits, tiles);
     for (int M : {1, 2, 3, 9, 17, 28, 31, 33, 60, 64, 200}) {
         for (long long ldc : {1LL, 64LL, 4096LL, 1LL << 24, (1LL << 30) - 1, 1LL << 30}) checkStore(M, ldc);
         // strides whose multiples fall just past the view's end, mod 2^32
