@@ -6,9 +6,11 @@
 //
 // Composed of a scale pass and, per head, a product, a softmax and a product, ViT-B/16 at batch 16
 // (197 tokens, 12 heads) took 37 launches of a few us each, 250 us, and passed the scores through
-// memory four times; its 1.9 GFLOP are 12 us of fp32 MFMA. This kernel takes 50 us: 13 of each head's 16
-// wave slots hold queries and the MFMAs wait on the softmax of their own wave (82 us with LDS reads
-// hoisted, which spilled). Here a workgroup of four waves holds 64
+// memory four times; its 1.9 GFLOP are 12 us of fp32 MFMA. This kernel takes 32 us (few
+// workgroups at hd 64: 4.6 us and 3.5 us more per 64 keys): 13 of each head's 16 wave slots hold queries and the
+// MFMAs wait on the softmax of their own wave. LDS reads hoisted to the front of a trip spilled (82 against 50
+// us), and context stores through a descriptor per lane were loops of one lane a turn (50 against 32 us; 16
+// tokens 14 against 4.6 us). Here a workgroup of four waves holds 64
 // queries of one head and walks the keys 64 at a time:
 //  * K and V rows pass memory -> registers -> LDS, the next 64 keys loading under this 64's math;
 //  * scores^T = K . Q^T with v_mfma_f32_16x16x4_f32. Lane (l16, g = lane / 16) supplies k = g of each
@@ -174,16 +176,18 @@ __global__ __launch_bounds__(kThreads, DT <= 4 ? 3 : 2) void attention_f32_kerne
     if (!active) return;
     sum += __shfl_xor(sum, 16, 64);
     sum += __shfl_xor(sum, 32, 64);
-    const int row = qb * kQueries + wave * 16 + l16;
-    if (row >= p.S) return;
-    float* const op = p.out + ((long long)b * p.S + row) * p.ldo + (long long)h * p.hd;
+    // One view of the block's rows: a descriptor is uniform over a wave (from one per lane the compiler makes a
+    // loop that stores a lane a turn).
+    const int rows = min(kQueries, p.S - qb * kQueries), row = wave * 16 + l16;
+    const uint32_t ldo4 = (uint32_t)p.ldo * 4u;
+    const auto w = bufferRsrc(p.out + ((long long)b * p.S + qb * kQueries) * p.ldo + (long long)h * p.hd,
+                              (uint32_t)(rows - 1) * ldo4 + rowBytes);
 #pragma unroll
     for (int i = 0; i < DT; ++i) {
         const int d = 16 * i + 4 * g;
-        if (d >= p.hd) continue;
         const f32x4 v = o[i] / sum;
-        const auto w = bufferRsrc(op + d, 16u);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4s, v), w, 0, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4s, v), w,
+                                               row < rows && d < p.hd ? row * ldo4 + d * 4u : kOOB, 0, 0);
     }
 }
 

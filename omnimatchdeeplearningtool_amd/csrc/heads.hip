@@ -297,7 +297,7 @@ int omHipAttention(const float* pQKV, float* pOut, int nBatch, int nSeq, int nHe
     const int outer = headsOuter ? nHeads : nBatch, inner = headsOuter ? nBatch : nHeads;
     if ((long long)inner * S * S > 0x7fffffffLL)
         return fail("%s: %d x %lld x %lld scores exceed the 2^31-element limit", name, inner, S, S);
-    // One kernel wherever it fits (ViT-B/16 b16: 250 us below, 50 us there); the rest takes products of any sizes.
+    // One kernel wherever it fits (ViT-B/16 b16: 250 us below, 32 us there); the rest takes products of any sizes.
     if (attentionF32Fits(nBatch, nSeq, nHeads, nHeadDim))
         return attentionF32(pQKV, pOut, nBatch, nSeq, nHeads, nHeadDim, fScale);
     const size_t bQ = up((size_t)(T * D) * 4), bScores = up((size_t)inner * S * S * 4);

@@ -109,6 +109,21 @@ def test_gemm_plan_partials_fit_the_fixed_scratch(tmp_path):
     assert r.returncode == 0 and "ALL PASSED" in r.stdout
 
 
+def test_attention_f32_stores_whole_waves(tmp_path):
+    """Every buffer access of the fp32 attention kernels has a descriptor that is uniform over the wave: the compiled
+    code holds no loop over lanes that compares descriptors."""
+    from omnimatchdeeplearningtool_amd import build as b
+    if not os.path.exists(b.HIPCC):
+        pytest.skip("hipcc not found")
+    out = tmp_path / "attention_f32.s"
+    src = "attention_f32.hip"
+    subprocess.run([b.HIPCC, f"--offload-arch={b.ARCH}", *b.COMMON, *b.DEVICE_FLAGS, *b.EXTRA_FLAGS[src], "--offload-device-only",
+                    "-S", os.path.join(b.CSRC, src), "-o", str(out)], check=True, stderr=subprocess.DEVNULL, timeout=300)
+    text = out.read_text()
+    assert text.count("buffer_store_dwordx4") >= 8
+    assert "v_cmp_eq_u64" not in text
+
+
 def test_bench_refuses_multi_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], stdout=subprocess.PIPE,
                        stderr=subprocess.PIPE, text=True, timeout=120)
