@@ -112,7 +112,7 @@ template <int BM, int BK, int NT, bool VEC>
 struct WeightLoader {
     static constexpr int PER_T = VEC ? BM * BK / 4 / NT : BM * BK / NT;
     static_assert(BM * BK % (NT * (VEC ? 4 : 1)) == 0, "slice must split evenly");
-    using Shape = LdsShape<true, BM, BK>;
+    using Shape = LdsShape<BM, BK>;
     __amdgpu_buffer_rsrc_t r;
     uint32_t voff[PER_T];
     f32x4 v4[VEC ? PER_T : 1];
@@ -183,7 +183,7 @@ struct GatherLoader {
     static constexpr int TPC = NT / BN;
     static constexpr int RPT = BK / TPC;
     static_assert(NT % BN == 0 && BK % TPC == 0 && BN >= 64 && RPT % 4 == 0, "gather mapping");
-    using Shape = LdsShape<true, BN, BK>;
+    using Shape = LdsShape<BN, BK>;
     __amdgpu_buffer_rsrc_t r;
     uint32_t voffPix;
     uint32_t invLo, invHi;
@@ -460,8 +460,8 @@ __device__ __forceinline__ void stageEpilogue(const ConvParams& p, float* sEpi, 
 template <class Cfg, bool VA, int MODE>
 __global__ __launch_bounds__(Cfg::NT) void conv_igemm_kernel(ConvParams p) {
     extern __shared__ float smem[];
-    using SA = LdsShape<true, Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<true, Cfg::BN, Cfg::BK>;
+    using SA = LdsShape<Cfg::BM, Cfg::BK>;
+    using SB = LdsShape<Cfg::BN, Cfg::BK>;
     constexpr int STAGE = SA::SIZE + SB::SIZE;
     float* sEpi = smem + 2 * STAGE;   // [5][BM]: bias, mean, invStd, gamma, beta
     int* sFlag = reinterpret_cast<int*>(sEpi + 5 * Cfg::BM);   // last-arrival flag of a split tile
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_igemm_kernel(ConvParams p) {
         lb2.template load<true>(kBeg + (t + 2) * Cfg::BK, tid);
         la2.template load<true>(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
         __builtin_amdgcn_sched_barrier(0);
-        mma_slice<Cfg, true, true>(smem, smem + SA::SIZE, acc, wm, wn, lane);
+        mma_slice<Cfg>(smem, smem + SA::SIZE, acc, wm, wn, lane);
         __builtin_amdgcn_sched_barrier(0);
         la.store(smem + STAGE, tid);
         lb.store(smem + STAGE + SA::SIZE, tid);
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_igemm_kernel(ConvParams p) {
         lb.template load<true>(kBeg + (t + 3) * Cfg::BK, tid);
         la.template load<true>(kBeg + (t + 3) * Cfg::BK, kEnd, tid);
         __builtin_amdgcn_sched_barrier(0);
-        mma_slice<Cfg, true, true>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
+        mma_slice<Cfg>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
         __builtin_amdgcn_sched_barrier(0);
         la2.store(smem, tid);
         lb2.store(smem + SA::SIZE, tid);
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_igemm_kernel(ConvParams p) {
             lb2.load(kBeg + (t + 2) * Cfg::BK, tid);
             la2.load(kBeg + (t + 2) * Cfg::BK, kEnd, tid);
         }
-        mma_slice<Cfg, true, true>(smem, smem + SA::SIZE, acc, wm, wn, lane);
+        mma_slice<Cfg>(smem, smem + SA::SIZE, acc, wm, wn, lane);
         if (t + 1 < nk) {
             la.store(smem + STAGE, tid);
             lb.store(smem + STAGE + SA::SIZE, tid);
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_igemm_kernel(ConvParams p) {
                 lb.load(kBeg + (t + 3) * Cfg::BK, tid);
                 la.load(kBeg + (t + 3) * Cfg::BK, kEnd, tid);
             }
-            mma_slice<Cfg, true, true>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
+            mma_slice<Cfg>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
             if (t + 2 < nk) {
                 la2.store(smem, tid);
                 lb2.store(smem + SA::SIZE, tid);
@@ -609,7 +609,7 @@ using ConvCfg = ConvCfgT<OMHIP_CONV_TILE>;
 template <class Cfg>
 static size_t convLds() {
     // two A+B stages and the epilogue vectors
-    return (2 * (LdsShape<true, Cfg::BM, Cfg::BK>::SIZE + LdsShape<true, Cfg::BN, Cfg::BK>::SIZE) + 5 * Cfg::BM + 4) *
+    return (2 * (LdsShape<Cfg::BM, Cfg::BK>::SIZE + LdsShape<Cfg::BN, Cfg::BK>::SIZE) + 5 * Cfg::BM + 4) *
            sizeof(float);
 }
 

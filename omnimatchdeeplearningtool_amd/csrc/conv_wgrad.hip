@@ -107,7 +107,7 @@ template <int R, int BK, int NT, bool VEC>
 struct PlaneLoader {
     static constexpr int PER_T = VEC ? R * BK / 4 / NT : R * BK / NT;
     static_assert(R * BK % (NT * (VEC ? 4 : 1)) == 0, "slice must split evenly");
-    using Shape = LdsShape<true, R, BK>;
+    using Shape = LdsShape<R, BK>;
     __amdgpu_buffer_rsrc_t r;
     uint32_t rowOff[PER_T];
     uint32_t mul, shift, step;
@@ -173,7 +173,7 @@ struct TapLoader {
     static constexpr int TPC = NT / BN;
     static constexpr int RPT = BK / TPC;
     static_assert(NT % BN == 0 && BK % TPC == 0 && BN >= 64 && RPT % 4 == 0, "tap loader mapping");
-    using Shape = LdsShape<true, BN, BK>;
+    using Shape = LdsShape<BN, BK>;
     __amdgpu_buffer_rsrc_t r;
     uint32_t tapOff;
     uint32_t tap;      // mask modes: kh*KW + kw
@@ -235,7 +235,7 @@ struct PixelLoader {
     static constexpr int CPT = BN * BK / NT;   // columns per thread
     static constexpr int CSTEP = NT / BK;
     static_assert(NT % BK == 0 && BN % CSTEP == 0, "pixel loader mapping");
-    using Shape = LdsShape<true, BN, BK>;
+    using Shape = LdsShape<BN, BK>;
     __amdgpu_buffer_rsrc_t r;
     uint32_t tapOff[CPT];
     uint32_t tap[CPT];
@@ -300,8 +300,8 @@ __device__ __forceinline__ void startLoader(L& l, int q0, int tid) {
 
 template <class Cfg, bool VA, int XK>
 __global__ __launch_bounds__(Cfg::NT) void conv_wgrad_kernel(WgradParams p) {
-    using SA = LdsShape<true, Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<true, Cfg::BN, Cfg::BK>;
+    using SA = LdsShape<Cfg::BM, Cfg::BK>;
+    using SB = LdsShape<Cfg::BN, Cfg::BK>;
     constexpr int STAGE = SA::SIZE + SB::SIZE;
     __shared__ __attribute__((aligned(16))) float smem[2 * STAGE];
 
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_wgrad_kernel(WgradParams p) {
                 lb.load(qBeg + (t + 1) * Cfg::BK, tid);
                 la.load(qBeg + (t + 1) * Cfg::BK, tid);
             }
-            mma_slice<Cfg, true, true>(smem, smem + SA::SIZE, acc, wm, wn, lane);
+            mma_slice<Cfg>(smem, smem + SA::SIZE, acc, wm, wn, lane);
             if (more) {
                 la.store(smem + STAGE, tid);
                 lb.store(smem + STAGE + SA::SIZE, tid);
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_wgrad_kernel(WgradParams p) {
                 lb.load(qBeg + (t + 2) * Cfg::BK, tid);
                 la.load(qBeg + (t + 2) * Cfg::BK, tid);
             }
-            mma_slice<Cfg, true, true>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
+            mma_slice<Cfg>(smem + STAGE, smem + STAGE + SA::SIZE, acc, wm, wn, lane);
             if (more) {
                 la.store(smem, tid);
                 lb.store(smem + SA::SIZE, tid);

@@ -14,10 +14,8 @@
 // this permutation only changes rounding order, and it lets an operand whose
 // K is contiguous be read from LDS 4 k at a time (ds_read_b128).
 //
-// Operand storage in LDS is chosen by the operand's layout in HBM:
-//   KMAJOR: element (r,k) at P[r*ld + k]   -> LDS [R][BK+4]   (b128 fragment reads)
-//   RMAJOR: element (r,k) at P[k*ld + r]   -> LDS [BK][R+4]   (b32 fragment reads)
-// where r is the M index for A and the N index for B.
+// Operands lie in LDS with K contiguous, [R][BK+4] floats, whatever their layout
+// in HBM (r is the M index for A and the N index for B; b128 fragment reads).
 //
 // Accumulator layout of a 32x32 block (lane l, register i):
 //   row = 8*(i/4) + 4*(l/32) + (i%4),  col = l%32.
@@ -44,22 +42,22 @@ struct TileCfg {
     static_assert(BK % 8 == 0, "BK must be a multiple of 8");
 };
 
-// LDS footprint (floats) of one buffer of an operand with R rows.
-template <bool KMAJOR, int R, int BK>
+// LDS row stride and footprint (floats) of one buffer of an operand with R rows.
+template <int R, int BK>
 struct LdsShape {
-    static constexpr int LD = KMAJOR ? (BK + 4) : (R + 4);
-    static constexpr int SIZE = KMAJOR ? R * (BK + 4) : BK * (R + 4);
+    static constexpr int LD = BK + 4;
+    static constexpr int SIZE = R * LD;
 };
 
 // ---------------------------------------------------------------------------
 // Fragment reads + MFMA over one LDS slice.
 // ---------------------------------------------------------------------------
-template <class Cfg, bool A_KMAJOR, bool B_KMAJOR>
+template <class Cfg>
 __device__ __forceinline__ void mma_slice(const float* __restrict__ sA, const float* __restrict__ sB,
                                           f32x16 (&acc)[Cfg::FM][Cfg::FN],
                                           int wm, int wn, int lane) {
-    using SA = LdsShape<A_KMAJOR, Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<B_KMAJOR, Cfg::BN, Cfg::BK>;
+    using SA = LdsShape<Cfg::BM, Cfg::BK>;
+    using SB = LdsShape<Cfg::BN, Cfg::BK>;
     const int li = lane & 31;
     const int h = lane >> 5;
     const int kb = h * Cfg::KH;
@@ -69,24 +67,14 @@ __device__ __forceinline__ void mma_slice(const float* __restrict__ sA, const fl
 #pragma unroll
         for (int fm = 0; fm < Cfg::FM; ++fm) {
             const int row = wm * Cfg::WM + fm * 32 + li;
-            if constexpr (A_KMAJOR) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(sA + row * SA::LD + kb + 4 * u);
-                a[fm][0] = v[0]; a[fm][1] = v[1]; a[fm][2] = v[2]; a[fm][3] = v[3];
-            } else {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) a[fm][s] = sA[(kb + 4 * u + s) * SA::LD + row];
-            }
+            const f32x4 v = *reinterpret_cast<const f32x4*>(sA + row * SA::LD + kb + 4 * u);
+            a[fm][0] = v[0]; a[fm][1] = v[1]; a[fm][2] = v[2]; a[fm][3] = v[3];
         }
 #pragma unroll
         for (int fn = 0; fn < Cfg::FN; ++fn) {
             const int col = wn * Cfg::WN + fn * 32 + li;
-            if constexpr (B_KMAJOR) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(sB + col * SB::LD + kb + 4 * u);
-                b[fn][0] = v[0]; b[fn][1] = v[1]; b[fn][2] = v[2]; b[fn][3] = v[3];
-            } else {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) b[fn][s] = sB[(kb + 4 * u + s) * SB::LD + col];
-            }
+            const f32x4 v = *reinterpret_cast<const f32x4*>(sB + col * SB::LD + kb + 4 * u);
+            b[fn][0] = v[0]; b[fn][1] = v[1]; b[fn][2] = v[2]; b[fn][3] = v[3];
         }
 #pragma unroll
         for (int s = 0; s < 4; ++s)
