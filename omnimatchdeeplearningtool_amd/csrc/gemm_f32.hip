@@ -111,50 +111,70 @@ __device__ __forceinline__ bool splitArrive(const GemmF32Params& p, f32x16 (&acc
     return true;
 }
 
-// acc = op(A) * op(B) over [kBeg, kEnd) for one wave's WM x WN block at (m0, n0)
-// on the fp32 MFMA, its fragments read from memory element by element behind
-// bounds tests: any stride and alignment, no LDS. It recomputes the blocks
-// whose operands the pieces cannot carry, and serves strides beyond the buffer
-// views' range.
-template <class Cfg, bool TA, bool TB>
-__device__ __forceinline__ void plainProduct(const GemmF32Params& p, f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0, int n0,
-                                             long long batch, int kBeg, int kEnd, int lane) {
-    const int li = lane & 31, h = lane >> 5;
-    const float* A = p.A + batch * p.sA;
-    const float* B = p.B + batch * p.sB;
+// acc = op(A) * op(B) over [kBeg, kEnd) on the fp32 MFMA: the tiles whose
+// operands the pieces cannot carry, and with FAR (64-bit addresses) strides
+// beyond the buffer views. Two slices are in flight: while slice t is multiplied
+// from LDS, slice t + 1, loaded one slice earlier, goes to the other stage and
+// slice t + 2 is loaded. smem: two stages of both operands' slices.
+template <class Cfg, bool TA, bool TB, bool FAR>
+__device__ __forceinline__ void plainLoop(const GemmF32Params& p, float* smem, f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0,
+                                          int n0, long long batch, int kBeg, int kEnd, int wm, int wn, int lane,
+                                          int tid) {
+    constexpr int OFF_B = LdsShape<Cfg::BM, 16>::SIZE, STAGE = OFF_B + LdsShape<Cfg::BN, 16>::SIZE;
+    using LA = std::conditional_t<FAR, FarLoader<!TA, Cfg::BM, Cfg::NT>, SplitLoader<!TA, Cfg::BM, Cfg::NT>>;
+    using LB = std::conditional_t<FAR, FarLoader<TB, Cfg::BN, Cfg::NT>, SplitLoader<TB, Cfg::BN, Cfg::NT>>;
+    LA la[2];
+    LB lb[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        la[j].init(p.A + batch * p.sA, p.lda, p.M, m0, tid);
+        lb[j].init(p.B + batch * p.sB, p.ldb, p.N, n0, tid);
+    }
 #pragma unroll
     for (int i = 0; i < Cfg::FM; ++i)
 #pragma unroll
         for (int j = 0; j < Cfg::FN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    // one 32x32 block at a time, so that few addresses are live beside the sums; rows and
-    // k past the end read the last one and count as zero
-#pragma unroll
-    for (int fm = 0; fm < Cfg::FM; ++fm)
-#pragma unroll
-        for (int fn = 0; fn < Cfg::FN; ++fn) {
-            const int r = m0 + fm * 32 + li, c = n0 + fn * 32 + li;
-            const float* pa = A + min(r, p.M - 1) * (TA ? 1 : p.lda);
-            const float* pb = B + min(c, p.N - 1) * (TB ? p.ldb : 1);
-            const long long da = TA ? p.lda : 1, db = TB ? 1 : p.ldb;
-#pragma unroll 1
-            for (int k0 = kBeg; k0 < kEnd; k0 += 16) {   // the lane halves take eight k each
-                float a[8], b[8];
-#pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    const long long k = min(k0 + 8 * h + s, kEnd - 1);
-                    a[s] = pa[k * da];
-                    b[s] = pb[k * db];
-                }
-#pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    const bool in = k0 + 8 * h + s < kEnd;
-                    acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && r < p.M ? a[s] : 0.f,
-                                                                       in && c < p.N ? b[s] : 0.f, acc[fm][fn], 0, 0, 0);
-                }
-            }
+    const int nk = (kEnd - kBeg + 15) / 16, nFull = (kEnd - kBeg) / 16;
+    la[0].template load<false>(kBeg, kEnd, tid);
+    lb[0].template load<false>(kBeg, kEnd, tid);
+    if (nk > 1) {
+        la[1].template load<false>(kBeg + 16, kEnd, tid);
+        lb[1].template load<false>(kBeg + 16, kEnd, tid);
+    }
+    la[0].storePlain(smem, tid);
+    lb[0].storePlain(smem + OFF_B, tid);
+    __syncthreads();
+    // FULL: slices t + 1 and t + 2 exist and are whole
+    auto step = [&](auto full, int t, int j) {
+        constexpr bool FULL = decltype(full)::value;
+        if (FULL || t + 2 < nk) {
+            la[j].template load<FULL>(kBeg + (t + 2) * 16, kEnd, tid);
+            lb[j].template load<FULL>(kBeg + (t + 2) * 16, kEnd, tid);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        const float* cur = smem + j * STAGE;
+        float* oth = smem + (j ^ 1) * STAGE;
+        mma_slice_split<Cfg>(cur, cur + OFF_B, acc, wm, wn, lane, [&] {
+            if (FULL || t + 1 < nk) {
+                la[j ^ 1].storePlain(oth, tid);
+                lb[j ^ 1].storePlain(oth + OFF_B, tid);
+            }
+        });
+        __syncthreads();
+    };
+    int t = 0;
+#pragma unroll 1
+    for (; t + 3 < nFull; t += 2) {
+        step(std::true_type{}, t, 0);
+        step(std::true_type{}, t + 1, 1);
+    }
+#pragma unroll 1
+    for (; t < nk; t += 2) {
+        step(std::false_type{}, t, 0);
+        if (t + 1 < nk) step(std::false_type{}, t + 1, 1);
+    }
 }
 
 // 16-deep slices per LDS stage, and so per block barrier. The 64x64 tile has six
@@ -163,11 +183,15 @@ __device__ __forceinline__ void plainProduct(const GemmF32Params& p, f32x16 (&ac
 template <class Cfg>
 constexpr int kSub = Cfg::FM * Cfg::FN == 1 ? 2 : 1;
 
-// LDS: two stages of both operands' pieces.
+// LDS: two stages of both operands' pieces; the fp32 MFMA's loop uses the same.
 template <class Cfg>
 constexpr int kSliceBytes = SplitLds<Cfg::BM>::SIZE + SplitLds<Cfg::BN>::SIZE;
 template <class Cfg>
-constexpr size_t ldsBytes() { return 2 * kSub<Cfg> * kSliceBytes<Cfg>; }
+constexpr size_t ldsBytes() {
+    static_assert(kSliceBytes<Cfg> >= (int)sizeof(float) * (LdsShape<Cfg::BM, 16>::SIZE + LdsShape<Cfg::BN, 16>::SIZE),
+                  "the fp32 MFMA's slices fit the pieces'");
+    return 2 * kSub<Cfg> * kSliceBytes<Cfg>;
+}
 
 // The main loop of one tile: stage T & 1 (SUB slices) is multiplied from LDS
 // while stage T + 1 goes from its registers to the other half of LDS and stage
@@ -262,7 +286,14 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
 // op(A) * op(B). GATE: each element of C is kept where p.gate (same shape, row
 // stride p.ldg) is > 0 and set to 0 elsewhere (a ReLU's backward applied to the
 // product). PLAIN: on the fp32 MFMA from the start (strides beyond the buffer
-// views). Every tile adds a product's terms in the same order.
+// views). A tile in which any sum is not finite is computed again on the fp32
+// MFMA, whole, so the last bits of its finite elements depend on such neighbours
+// (and on which tile the plan chose); where all sums of a tile are finite, every
+// tile adds a product's terms in the same order.
+// Computing again costs that unit's time after the pieces': 4096^3 with one NaN
+// element 1489 us, with NaN in every element 1379 (563 without, 952 on the fp32
+// MFMA alone); 1024^3 26.8 and 36.5 (20.8; 22.4). Read from memory by each wave
+// for its own block, without LDS, it took 3385, 5309, 58 and 91.
 template <class Cfg, bool TA, bool TB, bool PLAIN, bool GATE = false>
 __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, int bid, long long batch, int split) {
     static_assert(Cfg::BK == 16, "one MFMA step per slice");
@@ -317,13 +348,23 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
             }
     }
 
-    bool plain = PLAIN;
-    if constexpr (!PLAIN) {
+    if constexpr (PLAIN) {
+        plainLoop<Cfg, TA, TB, true>(p, reinterpret_cast<float*>(smem), acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
+    } else {
         splitLoop<Cfg, TA, TB>(p, smem, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
-        plain = __any(unscaleSums(acc));
+        int* const bad = reinterpret_cast<int*>(smem);   // a word per wave; the stages are free
+        const bool mine = __any(unscaleSums(acc));
+        if (lane == 0) bad[wave] = mine;
+        __syncthreads();
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < Cfg::NWAVES; ++w) any |= bad[w];
+        if (__builtin_amdgcn_readfirstlane(any)) {
+            __syncthreads();
+            plainLoop<Cfg, TA, TB, false>(p, reinterpret_cast<float*>(smem), acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane,
+                                          tid);
+        }
     }
-    if (plain)
-        plainProduct<Cfg, TA, TB>(p, acc, m0 + wm * Cfg::WM, n0 + wn * Cfg::WN, batch, kBeg, kEnd, lane);
 
     const int li = lane & 31, h = lane >> 5;
     if constexpr (Cfg::BM * Cfg::BN <= 64 * 64) {   // the plans split K over the small tile only

@@ -86,6 +86,51 @@ __device__ __forceinline__ void mma_slice(const float* __restrict__ sA, const fl
     }
 }
 
+// The MFMAs of one LDS slice with `mid` run between its first and second
+// halves: every fragment of the slice is read first, then the first half of
+// the k steps, mid() (the next slice's LDS stores), the second half. The
+// schedule barriers keep that order, so the stores' LDS traffic overlaps the
+// second half's MFMAs instead of sitting between the last MFMA and the block
+// barrier.
+template <class Cfg, class Mid>
+__device__ __forceinline__ void mma_slice_split(const float* __restrict__ sA, const float* __restrict__ sB,
+                                                f32x16 (&acc)[Cfg::FM][Cfg::FN], int wm, int wn, int lane,
+                                                Mid&& mid) {
+    using SA = LdsShape<Cfg::BM, Cfg::BK>;
+    using SB = LdsShape<Cfg::BN, Cfg::BK>;
+    constexpr int U = Cfg::KH / 4;
+    static_assert(U % 2 == 0, "two halves of k steps");
+    const int li = lane & 31;
+    const int h = lane >> 5;
+    const int kb = h * Cfg::KH;
+    f32x4 a[U][Cfg::FM], b[U][Cfg::FN];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int fm = 0; fm < Cfg::FM; ++fm)
+            a[u][fm] = *reinterpret_cast<const f32x4*>(sA + (wm * Cfg::WM + fm * 32 + li) * SA::LD + kb + 4 * u);
+#pragma unroll
+        for (int fn = 0; fn < Cfg::FN; ++fn)
+            b[u][fn] = *reinterpret_cast<const f32x4*>(sB + (wn * Cfg::WN + fn * 32 + li) * SB::LD + kb + 4 * u);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (u == U / 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            mid();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int fm = 0; fm < Cfg::FM; ++fm)
+#pragma unroll
+                for (int fn = 0; fn < Cfg::FN; ++fn)
+                    acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][fm][s], b[u][fn][s], acc[fm][fn], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // ---------------------------------------------------------------------------
 // Block-tile -> (tm, tn) mapping. Workgroups are dispatched round-robin over
 // the 8 XCDs (each with its own L2), so consecutive block ids land on

@@ -22,8 +22,9 @@
 // then every bit of every fp32 value down to the smallest denormal (2^-149)
 // lies in the pieces' range (2^-133). What the pieces cannot carry leaves a
 // non-finite sum in every output it takes part in (x - h of an infinite or NaN
-// h is NaN): infinities, NaN, |x| >= 2^111 and sums of 2^95 and more. A tile
-// with such a sum is recomputed on the fp32 MFMA.
+// h is NaN): infinities, NaN, |x| from 2^112 - 2^103 on (a scaled value that
+// rounds past the largest bf16) and sums of 2^96 and more. A tile with such a sum
+// is computed again on the fp32 MFMA.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -132,6 +133,14 @@ struct SplitLoaderK {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i) storePart(i, s, tid);
     }
+    // The slice as it is, for the fp32 MFMA.
+    __device__ __forceinline__ void storePlain(float* s, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PER_T; ++i) {
+            const int e = tid + i * NT;
+            *reinterpret_cast<f32x4*>(s + e / 4 * LdsShape<R, 16>::LD + e % 4 * 4) = v[i];
+        }
+    }
 };
 
 // Loader of an R-contiguous operand: element (r, k) at P[k * ld + r]. A thread
@@ -199,6 +208,52 @@ struct SplitLoaderR {
     __device__ __forceinline__ void store(char* s, int tid) {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i) storePart(i, s, tid);
+    }
+    __device__ __forceinline__ void storePlain(float* s, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
+            *reinterpret_cast<f32x4*>(s + tid % R * LdsShape<R, 16>::LD + tid / R * KU + 4 * i) =
+                f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+    }
+};
+
+// Loader of either layout by 64-bit addresses, for strides beyond the buffer
+// views: a thread's elements as above, one at a time.
+template <bool KMAJOR, int R, int NT>
+struct FarLoader {
+    static constexpr int KU = R * 16 / NT, UNITS = KU / 4;
+    const float* tile;
+    long long ld;
+    int rowsLeft;
+    f32x4 v[UNITS];
+
+    // Row and first k of the thread's i-th four elements.
+    static __device__ __forceinline__ int rowOf(int i, int tid) { return KMAJOR ? (tid + i * NT) / 4 : tid % R; }
+    static __device__ __forceinline__ int kOf(int i, int tid) {
+        return KMAJOR ? (tid + i * NT) % 4 * 4 : tid / R * KU + 4 * i;
+    }
+
+    __device__ __forceinline__ void init(const float* p, long long ld_, int rows, int r0, int) {
+        ld = ld_;
+        tile = KMAJOR ? p + r0 * ld : p + r0;
+        rowsLeft = rows - r0;
+    }
+    template <bool FULL>
+    __device__ __forceinline__ void load(int k0, int kEnd, int tid) {
+#pragma unroll
+        for (int i = 0; i < UNITS; ++i) {
+            const int r = rowOf(i, tid);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k = k0 + kOf(i, tid) + j;
+                v[i][j] = r < rowsLeft && (FULL || k < kEnd) ? tile[KMAJOR ? r * ld + k : k * ld + r] : 0.f;
+            }
+        }
+    }
+    __device__ __forceinline__ void storePlain(float* s, int tid) const {
+#pragma unroll
+        for (int i = 0; i < UNITS; ++i)
+            *reinterpret_cast<f32x4*>(s + rowOf(i, tid) * LdsShape<R, 16>::LD + kOf(i, tid)) = v[i];
     }
 };
 

@@ -80,7 +80,7 @@ def test_special_values(hip, layout, M, N, K):
     A[12, :] = 0
     A[12, 7] = np.inf                       # inf * b, and 0 elsewhere
     A[20, 4], B[4, 11] = 3.3e38, 1e-30      # beyond the pieces' range, finite products
-    A[21, 6] = -2.7e33                      # 2^111 and above
+    A[21, 6] = -2.7e33                      # 2^111
     B[6, :] *= np.float32(1e-20)
     A[30, :] = np.float32(1e-42)            # denormal
     A[31, :] = np.float32(3e-39)
@@ -113,6 +113,25 @@ def test_row_padding_is_not_read(hip, ta, tb, M, N):
             got.append(dC.numpy())
         assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
         assert _check(got[0], A, B, np.arange(M)).all()
+
+
+BF16_MAX = 2.0 ** 128 - 2.0 ** 120
+
+
+# The scaled operand's first piece overflows from half a bf16 ulp above the largest bf16 on (2^-16 of it, about
+# 2^112), a scaled sum at 2^128 (2^96 of the sum itself).
+@pytest.mark.parametrize("big,other", [(2.0 ** 111, 1e-3), (BF16_MAX * 2.0 ** -16, 1e-3), (2.0 ** 112 - 2.0 ** 103, 1e-3),
+                                       (2.0 ** 112, 1e-3), (3.4e38, 1e-3), (2.0 ** 94, 1.0), (2.0 ** 95, 1.0),
+                                       (2.0 ** 96, 1.0), (2.0 ** 97, 1.0), (2.0 ** 120, 2.0 ** -25), (2.0 ** 60, 2.0 ** 40)])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 33), (130, 70, 600), (2048, 2048, 20), (4096, 4096, 20)])
+def test_hand_over(hip, M, N, K, big, other):
+    """One huge element alone in the whole product, below and above what the pieces carry: its row is as exact as
+    any other, and so is the rest of its tile, which the fp32 MFMA computes again with it."""
+    print(f"case {M}x{N}x{K} {big:.3g}", flush=True)
+    A, B = _operands(M, N, K, 11)
+    A[5, K - 2] = big
+    B[K - 2, :] = (np.float32(other) * np.sign(B[K - 2, :])).astype(np.float32)
+    assert _check(_run(hip, "nn", A, B), A, B, np.r_[0:9, 30:36, 62:64]).all()
 
 
 @pytest.mark.parametrize("scale_a,scale_b", [(1e-42, 1e36), (1e-40, 1e-2), (1e-37, 1e-5), (1e32, 1e-32), (1e18, 1e19)])
