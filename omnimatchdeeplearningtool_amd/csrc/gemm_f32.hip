@@ -115,14 +115,17 @@ __device__ __forceinline__ bool splitArrive(const GemmF32Params& p, f32x16 (&acc
 // operands the pieces cannot carry, and with FAR (64-bit addresses) strides
 // beyond the buffer views. Two slices are in flight: while slice t is multiplied
 // from LDS, slice t + 1, loaded one slice earlier, goes to the other stage and
-// slice t + 2 is loaded. smem: two stages of both operands' slices.
-template <class Cfg, bool TA, bool TB, bool FAR>
+// slice t + 2 is loaded. smem: two stages of both operands' slices. VEC: the row
+// counts of the operands stored K first are multiples of four, and they are loaded
+// four rows at a time (with a test per load instead, 448 of K took 12.2 us for 11.2).
+template <class Cfg, bool TA, bool TB, bool FAR, bool VEC>
 __device__ __forceinline__ void plainLoop(const GemmF32Params& p, float* smem, f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0,
                                           int n0, long long batch, int kBeg, int kEnd, int wm, int wn, int lane,
                                           int tid) {
-    constexpr int OFF_B = LdsShape<Cfg::BM, 16>::SIZE, STAGE = OFF_B + LdsShape<Cfg::BN, 16>::SIZE;
-    using LA = std::conditional_t<FAR, FarLoader<!TA, Cfg::BM, Cfg::NT>, SplitLoader<!TA, Cfg::BM, Cfg::NT>>;
-    using LB = std::conditional_t<FAR, FarLoader<TB, Cfg::BN, Cfg::NT>, SplitLoader<TB, Cfg::BN, Cfg::NT>>;
+    using LA = PlainLoader<!TA, Cfg::BM, Cfg::NT, FAR, VEC>;
+    using LB = PlainLoader<TB, Cfg::BN, Cfg::NT, FAR, VEC>;
+    constexpr int OFF_B = LdsShape<Cfg::BM, 16, LA::PLAIN_KMAJOR>::SIZE;
+    constexpr int STAGE = OFF_B + LdsShape<Cfg::BN, 16, LB::PLAIN_KMAJOR>::SIZE;
     LA la[2];
     LB lb[2];
 #pragma unroll
@@ -156,7 +159,7 @@ __device__ __forceinline__ void plainLoop(const GemmF32Params& p, float* smem, f
         __builtin_amdgcn_sched_barrier(0);
         const float* cur = smem + j * STAGE;
         float* oth = smem + (j ^ 1) * STAGE;
-        mma_slice_split<Cfg>(cur, cur + OFF_B, acc, wm, wn, lane, [&] {
+        mma_slice_split<Cfg, LA::PLAIN_KMAJOR, LB::PLAIN_KMAJOR>(cur, cur + OFF_B, acc, wm, wn, lane, [&] {
             if (FULL || t + 1 < nk) {
                 la[j ^ 1].storePlain(oth, tid);
                 lb[j ^ 1].storePlain(oth + OFF_B, tid);
@@ -183,15 +186,8 @@ __device__ __forceinline__ void plainLoop(const GemmF32Params& p, float* smem, f
 template <class Cfg>
 constexpr int kSub = Cfg::FM * Cfg::FN == 1 ? 2 : 1;
 
-// LDS: two stages of both operands' pieces; the fp32 MFMA's loop uses the same.
 template <class Cfg>
 constexpr int kSliceBytes = SplitLds<Cfg::BM>::SIZE + SplitLds<Cfg::BN>::SIZE;
-template <class Cfg>
-constexpr size_t ldsBytes() {
-    static_assert(kSliceBytes<Cfg> >= (int)sizeof(float) * (LdsShape<Cfg::BM, 16>::SIZE + LdsShape<Cfg::BN, 16>::SIZE),
-                  "the fp32 MFMA's slices fit the pieces'");
-    return 2 * kSub<Cfg> * kSliceBytes<Cfg>;
-}
 
 // The main loop of one tile: stage T & 1 (SUB slices) is multiplied from LDS
 // while stage T + 1 goes from its registers to the other half of LDS and stage
@@ -282,11 +278,24 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
     }
 }
 
+// How a tile's products are computed: through the pieces, on the fp32 MFMA
+// (smallTilePlain), or on the fp32 MFMA with 64-bit addresses (strides beyond
+// the buffer views).
+enum class Path { Pieces, Plain, Far };
+
+// LDS: two stages of both operands' slices, as pieces or as they are; a tile of
+// the pieces that is computed again uses its stages for the plain slices.
+template <class Cfg, Path PATH>
+constexpr size_t ldsBytes() {
+    constexpr size_t plain = sizeof(float) * (LdsShape<Cfg::BM, 16>::SIZE + LdsShape<Cfg::BN, 16>::SIZE);
+    static_assert(kSliceBytes<Cfg> >= plain);
+    return 2 * (PATH == Path::Pieces ? kSub<Cfg> * kSliceBytes<Cfg> : plain);
+}
+
 // One output tile (bid: the tile's linear index, batch, split) of C =
 // op(A) * op(B). GATE: each element of C is kept where p.gate (same shape, row
 // stride p.ldg) is > 0 and set to 0 elsewhere (a ReLU's backward applied to the
-// product). PLAIN: on the fp32 MFMA from the start (strides beyond the buffer
-// views). A tile in which any sum is not finite is computed again on the fp32
+// product). A tile in which any sum is not finite is computed again on the fp32
 // MFMA, whole, so the last bits of its finite elements depend on such neighbours
 // (and on which tile the plan chose); where all sums of a tile are finite, every
 // tile adds a product's terms in the same order.
@@ -294,7 +303,7 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
 // element 1489 us, with NaN in every element 1379 (563 without, 952 on the fp32
 // MFMA alone); 1024^3 26.8 and 36.5 (20.8; 22.4). Read from memory by each wave
 // for its own block, without LDS, it took 3385, 5309, 58 and 91.
-template <class Cfg, bool TA, bool TB, bool PLAIN, bool GATE = false>
+template <class Cfg, bool TA, bool TB, Path PATH, bool GATE = false>
 __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, int bid, long long batch, int split) {
     static_assert(Cfg::BK == 16, "one MFMA step per slice");
     const int tid = threadIdx.x;
@@ -348,8 +357,19 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
             }
     }
 
-    if constexpr (PLAIN) {
-        plainLoop<Cfg, TA, TB, true>(p, reinterpret_cast<float*>(smem), acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
+    auto plain = [&] {
+        float* const s = reinterpret_cast<float*>(smem);
+        if constexpr (PATH == Path::Far) {
+            plainLoop<Cfg, TA, TB, true, false>(p, s, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
+        } else {
+            if ((TA || !TB) && (!TA || p.M % 4 == 0) && (TB || p.N % 4 == 0))
+                plainLoop<Cfg, TA, TB, false, true>(p, s, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
+            else
+                plainLoop<Cfg, TA, TB, false, false>(p, s, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
+        }
+    };
+    if constexpr (PATH != Path::Pieces) {
+        plain();
     } else {
         splitLoop<Cfg, TA, TB>(p, smem, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
         int* const bad = reinterpret_cast<int*>(smem);   // a word per wave; the stages are free
@@ -361,8 +381,7 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
         for (int w = 0; w < Cfg::NWAVES; ++w) any |= bad[w];
         if (__builtin_amdgcn_readfirstlane(any)) {
             __syncthreads();
-            plainLoop<Cfg, TA, TB, false>(p, reinterpret_cast<float*>(smem), acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane,
-                                          tid);
+            plain();
         }
     }
 
@@ -374,7 +393,7 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
     }
     // A lane's 16 rows of a block are 8 (r / 4) + r % 4 past its first one: a wave-uniform
     // byte offset past its own. Rows and columns past the matrix get an offset out of the
-    // view's range and store nothing. (PLAIN: ldc may be beyond the view, 64-bit addresses.)
+    // view's range and store nothing. (Far: ldc may be beyond the view, 64-bit addresses.)
     float* C = p.C + batch * p.sC + (long long)m0 * p.ldc + n0;
     const auto rc = bufferRsrc(C, kSplitView);
     const bool bias = p.bias != nullptr;
@@ -399,7 +418,7 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
                 if (relu) v = v > 0.f ? v : 0.f;
                 if constexpr (GATE) v = gatev[fm][fn][r] > 0.f ? v : 0.f;
                 const bool in = colOk && m0 + rl + ro < p.M;
-                if constexpr (PLAIN) {
+                if constexpr (PATH == Path::Far) {
                     if (in) C[(long long)(rl + ro) * p.ldc + cl] = v;
                 } else {
                     bufStore1(rc, in ? voff : kSplitOOB, storeRowOffset(ro, rowsLeft, p.ldc), v);
@@ -409,16 +428,16 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
     }
 }
 
-template <class Cfg, bool TA, bool TB, bool PLAIN>
+template <class Cfg, bool TA, bool TB, Path PATH>
 __global__ __launch_bounds__(Cfg::NT, 2) void gemm_f32_kernel(GemmF32Params p) {
     extern __shared__ __align__(16) char smem[];
-    gemmF32Tile<Cfg, TA, TB, PLAIN>(p, smem, blockIdx.x, blockIdx.z, blockIdx.y);
+    gemmF32Tile<Cfg, TA, TB, PATH>(p, smem, blockIdx.x, blockIdx.z, blockIdx.y);
 }
 
-template <class Cfg, bool TA, bool TB, bool PLAIN>
+template <class Cfg, bool TA, bool TB, Path PATH>
 static int launchOne(const GemmF32Params& prm, int batch, int splits) {
-    auto kern = gemm_f32_kernel<Cfg, TA, TB, PLAIN>;
-    constexpr size_t lds = ldsBytes<Cfg>();
+    auto kern = gemm_f32_kernel<Cfg, TA, TB, PATH>;
+    constexpr size_t lds = ldsBytes<Cfg, PATH>();
     OMHIP_CHECK(OMHIP_SET_MAX_DYNAMIC_LDS_ONCE(kern, lds));
     dim3 grid(prm.tilesM * prm.tilesN, splits, batch);
     hipLaunchKernelGGL(kern, grid, dim3(Cfg::NT), lds, stream(), prm);
@@ -446,27 +465,30 @@ using CfgM = TileCfg<128, 128, 16, 64, 64>;
 using CfgS = TileCfg<64, 64, 16, 32, 32>;
 
 template <class Cfg, bool TA, bool TB>
-static int launchTile(GemmF32Params prm, int batch, int splits) {
+static int launchTile(GemmF32Params prm, int batch, int splits, bool plain) {
     prm.tilesM = (prm.M + Cfg::BM - 1) / Cfg::BM;
     prm.tilesN = (prm.N + Cfg::BN - 1) / Cfg::BN;
     if (splitViewOk(!TA, Cfg::BM, prm.M, prm.lda) && splitViewOk(TB, Cfg::BN, prm.N, prm.ldb) &&
-        splitViewOk(true, Cfg::BM, prm.M, prm.ldc + Cfg::BN))
-        return launchOne<Cfg, TA, TB, false>(prm, batch, splits);
+        splitViewOk(true, Cfg::BM, prm.M, prm.ldc + Cfg::BN)) {
+        if constexpr (Cfg::BM == CfgS::BM)
+            if (plain) return launchOne<Cfg, TA, TB, Path::Plain>(prm, batch, splits);
+        return launchOne<Cfg, TA, TB, Path::Pieces>(prm, batch, splits);
+    }
     prm.tilesM = (prm.M + CfgS::BM - 1) / CfgS::BM;
     prm.tilesN = (prm.N + CfgS::BN - 1) / CfgS::BN;
-    return launchOne<CfgS, TA, TB, true>(prm, batch, splits);
+    return launchOne<CfgS, TA, TB, Path::Far>(prm, batch, splits);
 }
 
 // Tile and split-K choice (planGemmFor in gemm_f32.hpp) for this device.
-static GemmPlan planGemm(int M, int N, int K, int batch, bool wsOk) {
-    return planGemmFor(M, N, K, batch, wsOk, cuCount());
+static GemmPlan planGemm(bool ta, bool tb, int M, int N, int K, int batch, bool wsOk) {
+    return planGemmFor(M, N, K, batch, wsOk, cuCount(), ta, tb);
 }
 
 template <bool TA, bool TB>
-static int launchCfg(const GemmF32Params& prm, int batch, int splits, int cfg) {
-    if (cfg == 0) return launchTile<CfgL, TA, TB>(prm, batch, splits);
-    if (cfg == 1) return launchTile<CfgM, TA, TB>(prm, batch, splits);
-    return launchTile<CfgS, TA, TB>(prm, batch, splits);
+static int launchCfg(const GemmF32Params& prm, int batch, int splits, const GemmPlan& plan) {
+    if (plan.cfg == 0) return launchTile<CfgL, TA, TB>(prm, batch, splits, false);
+    if (plan.cfg == 1) return launchTile<CfgM, TA, TB>(prm, batch, splits, false);
+    return launchTile<CfgS, TA, TB>(prm, batch, splits, plan.plain);
 }
 
 // Launches the GEMM (split-K: partials to ws, summed in the same launch by
@@ -500,10 +522,10 @@ static int gemmF32Run(bool ta, bool tb, int batch, int M, int N, int K, const fl
         }
     }
     int rc;
-    if (!ta && !tb) rc = launchCfg<false, false>(prm, batch, splits, plan.cfg);
-    else if (!ta && tb) rc = launchCfg<false, true>(prm, batch, splits, plan.cfg);
-    else if (ta && !tb) rc = launchCfg<true, false>(prm, batch, splits, plan.cfg);
-    else rc = launchCfg<true, true>(prm, batch, splits, plan.cfg);
+    if (!ta && !tb) rc = launchCfg<false, false>(prm, batch, splits, plan);
+    else if (!ta && tb) rc = launchCfg<false, true>(prm, batch, splits, plan);
+    else if (ta && !tb) rc = launchCfg<true, false>(prm, batch, splits, plan);
+    else rc = launchCfg<true, true>(prm, batch, splits, plan);
     return rc;
 }
 
@@ -515,7 +537,7 @@ int gemmF32(bool ta, bool tb, int batch, int M, int N, int K,
             const float* B, long long ldb, long long sB,
             float* C, long long ldc, long long sC, const float* bias, int act) {
     const bool wsOk = (size_t)64 * batch * M * N * sizeof(float) <= kMaxSplitWorkspace;
-    const GemmPlan plan = planGemm(M, N, K, batch, wsOk);
+    const GemmPlan plan = planGemm(ta, tb, M, N, K, batch, wsOk);
     return gemmF32Run(ta, tb, batch, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, plan, bias, act);
 }
 
@@ -580,23 +602,23 @@ __device__ __forceinline__ void columnSum(const float* G, float* colSum, int row
 
 constexpr int kSumCols = 64;   // columns per workgroup of the sums: many workgroups, one wave each
 
-template <bool PLAIN, bool GATE>
+template <Path PATHW, Path PATHX, bool GATE>
 __global__ __launch_bounds__(CfgS::NT) void linear_backward_kernel(GemmF32Params pw, GemmF32Params pa, int tilesW,
                                                                   int tilesX, float* db) {
     extern __shared__ __align__(16) char smem[];
     const int b = blockIdx.x;
     if (b < tilesW)
-        gemmF32Tile<CfgS, true, false, PLAIN>(pw, smem, b, 0, 0);
+        gemmF32Tile<CfgS, true, false, PATHW>(pw, smem, b, 0, 0);
     else if (b < tilesW + tilesX)
-        gemmF32Tile<CfgS, false, true, PLAIN, GATE>(pa, smem, b - tilesW, 0, 0);
+        gemmF32Tile<CfgS, false, true, PATHX, GATE>(pa, smem, b - tilesW, 0, 0);
     else if (threadIdx.x < kSumCols)
         columnSum(pw.B, db, pw.K, pw.N, (b - tilesW - tilesX) * kSumCols + threadIdx.x);
 }
 
-template <bool PLAIN, bool GATE>
+template <Path PATHW, Path PATHX, bool GATE>
 static int launchLinearBackward(const GemmF32Params& pw, const GemmF32Params& pa, int tilesW, int tilesX, float* db) {
-    auto kern = linear_backward_kernel<PLAIN, GATE>;
-    constexpr size_t lds = ldsBytes<CfgS>();
+    auto kern = linear_backward_kernel<PATHW, PATHX, GATE>;
+    constexpr size_t lds = std::max(ldsBytes<CfgS, PATHW>(), ldsBytes<CfgS, PATHX>());
     OMHIP_CHECK(OMHIP_SET_MAX_DYNAMIC_LDS_ONCE(kern, lds));
     const int sums = db ? (pw.N + kSumCols - 1) / kSumCols : 0;
     hipLaunchKernelGGL(kern, dim3(tilesW + tilesX + sums), dim3(CfgS::NT), lds, stream(), pw, pa,
@@ -622,11 +644,18 @@ static int linearBackward(const float* X, const float* G, const float* W, const 
     const bool views = splitViewOk(false, CfgS::BM, I, I) && splitViewOk(false, CfgS::BN, O, O) &&
                        splitViewOk(true, CfgS::BM, B, O) && splitViewOk(true, CfgS::BN, I, O) &&
                        splitViewOk(true, CfgS::BM, B, I + CfgS::BN);
-    if (views)
-        return gate ? launchLinearBackward<false, true>(pw, pa, (int)tilesW, (int)tilesX, db)
-                    : launchLinearBackward<false, false>(pw, pa, (int)tilesW, (int)tilesX, db);
-    return gate ? launchLinearBackward<true, true>(pw, pa, (int)tilesW, (int)tilesX, db)
-                : launchLinearBackward<true, false>(pw, pa, (int)tilesW, (int)tilesX, db);
+    auto launch = [&](auto w, auto x) {
+        constexpr Path PW = decltype(w)::value, PX = decltype(x)::value;
+        return gate ? launchLinearBackward<PW, PX, true>(pw, pa, (int)tilesW, (int)tilesX, db)
+                    : launchLinearBackward<PW, PX, false>(pw, pa, (int)tilesW, (int)tilesX, db);
+    };
+    using Pieces = std::integral_constant<Path, Path::Pieces>;
+    using Plain = std::integral_constant<Path, Path::Plain>;
+    using Far = std::integral_constant<Path, Path::Far>;
+    if (!views) return launch(Far{}, Far{});
+    const bool plainW = smallTilePlain(tilesW, B, B, true, false, cuCount()), plainX = !dX || smallTilePlain(tilesX, O, O, false, true, cuCount());
+    if (plainW) return plainX ? launch(Plain{}, Plain{}) : launch(Plain{}, Pieces{});
+    return plainX ? launch(Pieces{}, Plain{}) : launch(Pieces{}, Pieces{});
 }
 
 // ---- fixed scratch of the no-allocation entry ---------------------------------
@@ -804,7 +833,7 @@ int omHipGemmStridedBatchedNoAlloc(int bTransA, int bTransB, int nBatch, int nM,
     if (!ws) return -1;
     // the same plan as omHipGemmStridedBatched, so the results are the same bits
     const bool wsOk = (size_t)64 * nBatch * nM * nN * sizeof(float) <= kMaxSplitWorkspace;
-    const GemmPlan plan = planGemm(nM, nN, nK, nBatch, wsOk);
+    const GemmPlan plan = planGemm(bTransA != 0, bTransB != 0, nM, nN, nK, nBatch, wsOk);
     auto run = [&] {
         return gemmF32Run(bTransA != 0, bTransB != 0, nBatch, nM, nN, nK, pA, nLda, nStrideA, pB, nLdb, nStrideB, pC,
                           nLdc, nStrideC, plan, nullptr, 0, ws, kNoAllocScratchBytes);

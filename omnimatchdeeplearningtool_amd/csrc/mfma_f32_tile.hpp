@@ -14,8 +14,9 @@
 // this permutation only changes rounding order, and it lets an operand whose
 // K is contiguous be read from LDS 4 k at a time (ds_read_b128).
 //
-// Operands lie in LDS with K contiguous, [R][BK+4] floats, whatever their layout
-// in HBM (r is the M index for A and the N index for B; b128 fragment reads).
+// Operands lie in LDS with K contiguous, [R][BK+4] floats (r is the M index for
+// A and the N index for B; b128 fragment reads), or, as mma_slice_split also takes
+// them, as [BK][R+4] (b32 fragment reads).
 //
 // Accumulator layout of a 32x32 block (lane l, register i):
 //   row = 8*(i/4) + 4*(l/32) + (i%4),  col = l%32.
@@ -42,11 +43,12 @@ struct TileCfg {
     static_assert(BK % 8 == 0, "BK must be a multiple of 8");
 };
 
-// LDS row stride and footprint (floats) of one buffer of an operand with R rows.
-template <int R, int BK>
+// LDS row stride and footprint (floats) of one buffer of an operand with R rows,
+// K contiguous or R contiguous.
+template <int R, int BK, bool KMAJOR = true>
 struct LdsShape {
-    static constexpr int LD = BK + 4;
-    static constexpr int SIZE = R * LD;
+    static constexpr int LD = KMAJOR ? BK + 4 : R + 4;
+    static constexpr int SIZE = KMAJOR ? R * LD : BK * LD;
 };
 
 // ---------------------------------------------------------------------------
@@ -92,26 +94,29 @@ __device__ __forceinline__ void mma_slice(const float* __restrict__ sA, const fl
 // schedule barriers keep that order, so the stores' LDS traffic overlaps the
 // second half's MFMAs instead of sitting between the last MFMA and the block
 // barrier.
-template <class Cfg, class Mid>
+template <class Cfg, bool A_KMAJOR, bool B_KMAJOR, class Mid>
 __device__ __forceinline__ void mma_slice_split(const float* __restrict__ sA, const float* __restrict__ sB,
                                                 f32x16 (&acc)[Cfg::FM][Cfg::FN], int wm, int wn, int lane,
                                                 Mid&& mid) {
-    using SA = LdsShape<Cfg::BM, Cfg::BK>;
-    using SB = LdsShape<Cfg::BN, Cfg::BK>;
+    using SA = LdsShape<Cfg::BM, Cfg::BK, A_KMAJOR>;
+    using SB = LdsShape<Cfg::BN, Cfg::BK, B_KMAJOR>;
     constexpr int U = Cfg::KH / 4;
     static_assert(U % 2 == 0, "two halves of k steps");
     const int li = lane & 31;
     const int h = lane >> 5;
     const int kb = h * Cfg::KH;
+    // four k of one row
+    auto fragment = [](const float* s, int ld, int row, int k, bool kMajor) {
+        if (kMajor) return *reinterpret_cast<const f32x4*>(s + row * ld + k);
+        return f32x4{s[k * ld + row], s[(k + 1) * ld + row], s[(k + 2) * ld + row], s[(k + 3) * ld + row]};
+    };
     f32x4 a[U][Cfg::FM], b[U][Cfg::FN];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
-        for (int fm = 0; fm < Cfg::FM; ++fm)
-            a[u][fm] = *reinterpret_cast<const f32x4*>(sA + (wm * Cfg::WM + fm * 32 + li) * SA::LD + kb + 4 * u);
+        for (int fm = 0; fm < Cfg::FM; ++fm) a[u][fm] = fragment(sA, SA::LD, wm * Cfg::WM + fm * 32 + li, kb + 4 * u, A_KMAJOR);
 #pragma unroll
-        for (int fn = 0; fn < Cfg::FN; ++fn)
-            b[u][fn] = *reinterpret_cast<const f32x4*>(sB + (wn * Cfg::WN + fn * 32 + li) * SB::LD + kb + 4 * u);
+        for (int fn = 0; fn < Cfg::FN; ++fn) b[u][fn] = fragment(sB, SB::LD, wn * Cfg::WN + fn * 32 + li, kb + 4 * u, B_KMAJOR);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {

@@ -75,7 +75,7 @@ struct SplitLds {
 // Loader of a K-contiguous operand: element (r, k) at P[r * ld + k], in
 // 4-float vectors (any 4-byte alignment). Per-lane byte offsets are fixed for
 // the K walk and each slice re-bases the buffer view; rows past the matrix read
-// zeros. Slices that end past kEnd load element by element. In-tile offsets
+// zeros. Slices that end past kEnd load element by element unless kEnd is a multiple of four. In-tile offsets
 // must stay below kSplitView (splitViewOk).
 template <int R, int NT>
 struct SplitLoaderK {
@@ -103,6 +103,8 @@ struct SplitLoaderK {
         const auto rs = bufferRsrc(tile + k0, kSplitView);
         if (FULL || k0 + Lds::BK <= kEnd) {
             v[i] = bufLoad4(rs, voff[i], 0);
+        } else if (kEnd % 4 == 0) {   // whole vectors inside or past the end
+            v[i] = bufLoad4(rs, k0 + ((tid + i * NT) % 4) * 4 < kEnd ? voff[i] : kSplitOOB, 0);
         } else {
             const int k = k0 + ((tid + i * NT) % 4) * 4;
 #pragma unroll
@@ -133,7 +135,8 @@ struct SplitLoaderK {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i) storePart(i, s, tid);
     }
-    // The slice as it is, for the fp32 MFMA.
+    // The slice as it is, for the fp32 MFMA: [R][16 + 4] (PLAIN_KMAJOR) or [16][R + 4].
+    static constexpr bool PLAIN_KMAJOR = true;
     __device__ __forceinline__ void storePlain(float* s, int tid) const {
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
@@ -209,6 +212,7 @@ struct SplitLoaderR {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i) storePart(i, s, tid);
     }
+    static constexpr bool PLAIN_KMAJOR = true;
     __device__ __forceinline__ void storePlain(float* s, int tid) const {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i)
@@ -217,8 +221,46 @@ struct SplitLoaderR {
     }
 };
 
-// Loader of either layout by 64-bit addresses, for strides beyond the buffer
-// views: a thread's elements as above, one at a time.
+// Loader of an R-contiguous operand for the fp32 MFMA whose row count is a
+// multiple of four: four consecutive rows of one k in a 16-byte word (any 4-byte
+// alignment), as they lie in memory.
+template <int R, int NT>
+struct PlainLoaderR {
+    static constexpr int PER_T = R * 4 / NT;
+    static_assert(R * 4 % NT == 0, "slice must divide over the threads");
+    const float* tile;
+    long long ld;
+    uint32_t voff[PER_T];
+    f32x4 v[PER_T];
+
+    __device__ __forceinline__ void init(const float* p, long long ld_, int rows, int r0, int tid) {
+        ld = ld_;
+        tile = p + r0;
+#pragma unroll
+        for (int i = 0; i < PER_T; ++i) {
+            const int e = tid + i * NT, r = e % (R / 4) * 4, k = e / (R / 4);
+            voff[i] = r0 + r < rows ? (uint32_t)((k * ld + r) * 4) : kSplitOOB;
+        }
+    }
+    template <bool FULL>
+    __device__ __forceinline__ void load(int k0, int kEnd, int tid) {
+        const auto rs = bufferRsrc(tile + (long long)k0 * ld, kSplitView);
+#pragma unroll
+        for (int i = 0; i < PER_T; ++i)
+            v[i] = bufLoad4(rs, FULL || k0 + (tid + i * NT) / (R / 4) < kEnd ? voff[i] : kSplitOOB, 0);
+    }
+    static constexpr bool PLAIN_KMAJOR = false;
+    __device__ __forceinline__ void storePlain(float* s, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PER_T; ++i) {
+            const int e = tid + i * NT;
+            *reinterpret_cast<f32x4*>(s + e / (R / 4) * LdsShape<R, 16, false>::LD + e % (R / 4) * 4) = v[i];
+        }
+    }
+};
+
+// Loader of either layout by 64-bit addresses, one element at a time, for strides
+// beyond the buffer views.
 template <bool KMAJOR, int R, int NT>
 struct FarLoader {
     static constexpr int KU = R * 16 / NT, UNITS = KU / 4;
@@ -250,6 +292,7 @@ struct FarLoader {
             }
         }
     }
+    static constexpr bool PLAIN_KMAJOR = true;
     __device__ __forceinline__ void storePlain(float* s, int tid) const {
 #pragma unroll
         for (int i = 0; i < UNITS; ++i)
@@ -262,6 +305,11 @@ constexpr int kSideValu = 26;
 
 template <bool KMAJOR, int R, int NT>
 using SplitLoader = std::conditional_t<KMAJOR, SplitLoaderK<R, NT>, SplitLoaderR<R, NT>>;
+
+// The fp32 MFMA's loaders. VEC: the rows of R-contiguous operands are multiples of four.
+template <bool KMAJOR, int R, int NT, bool FAR, bool VEC>
+using PlainLoader = std::conditional_t<FAR, FarLoader<KMAJOR, R, NT>,
+                                       std::conditional_t<KMAJOR || !VEC, SplitLoader<KMAJOR, R, NT>, PlainLoaderR<R, NT>>>;
 
 template <int R>
 __device__ __forceinline__ void readSplit(const char* s, int row, int half, bf16x8 (&f)[3]) {

@@ -17,6 +17,17 @@ static int g_fail = 0;
 static long long g_maxBytes = 0;
 
 static void check(int M, int N, int K, int batch, long long cus) {
+    // the layouts share tile and splits and differ in the unit that computes a small tile alone; sums of one
+    // product are always the fp32 MFMA's
+    for (int l = 0; l < 4; ++l) {
+        const omhip::GemmPlan a = omhip::planGemmFor(M, N, K, batch, true, cus, l & 1, l & 2);
+        const omhip::GemmPlan b = omhip::planGemmFor(M, N, K, batch, true, cus);
+        const omhip::GemmPlan one = omhip::planGemmFor(M, N, 1, batch, true, cus, l & 1, l & 2);
+        if (a.cfg != b.cfg || a.splits != b.splits || (a.plain && a.cfg != 2) || one.cfg != 2 || !one.plain) {
+            std::printf("FAIL layout %d M=%d N=%d K=%d batch=%d cus=%lld\n", l, M, N, K, batch, cus);
+            ++g_fail;
+        }
+    }
     // the wsOk rule of gemmF32: 64 splits of the batch's C within 256 MiB
     const bool wsOk = (long long)64 * batch * M * N * 4 <= (256LL << 20);
     const omhip::GemmPlan p = omhip::planGemmFor(M, N, K, batch, wsOk, cus);

@@ -71,6 +71,26 @@ def test_tile_edges(hip, layout, M, N):
         assert _check(_run(hip, layout, A, B), A, B, _rows(M)).all()
 
 
+# The plan's lines between the pieces and the fp32 MFMA on the 64x64 tile: few tiles (unsplit, split into short and
+# long pieces), more tiles than CUs; row counts that are and are not multiples of four; the last slice of each length.
+ROUTES = [(64, 60, k) for k in (1, 2, 3, 4, 5, 19, 31, 32, 33, 36, 511, 512, 530, 1000, 1023, 1024, 1030, 2047, 2048, 4100)] + \
+         [(61, 131, k) for k in (1, 3, 18, 47, 512, 1023, 1025, 2050)] + [(9, 4096, k) for k in (2040, 4099)] + \
+         [(1000, 2047, k) for k in (1, 30, 33, 191, 192, 193, 224, 288, 319, 320, 321, 322, 323, 338, 352)] + \
+         [(1500, 1501, k) for k in (32, 33, 127, 128, 129)]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N", sorted({r[:2] for r in ROUTES}))
+def test_small_tile_routes(hip, layout, M, N):
+    for K in [r[2] for r in ROUTES if r[:2] == (M, N)]:
+        print(f"case {layout} {M}x{N}x{K}", flush=True)
+        A, B = _operands(M, N, K, M + K)
+        got = _run(hip, layout, A, B)
+        assert _check(got, A, B, _rows(M)).all()
+        if K == 1:   # one product: the nearest float, in any layout
+            assert np.array_equal(got.view(np.uint32), (A * B).view(np.uint32))
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
 @pytest.mark.parametrize("M,N,K", [(70, 67, 40), (128, 256, 2048), (2048, 2048, 50), (2048, 4096, 50), (4096, 4096, 50)])
 def test_special_values(hip, layout, M, N, K):
