@@ -7,12 +7,21 @@
 // slice of K: al bh, ah bl, am bm, am bh, ah bm, ah bh. The three left out
 // are together below 2^-24 |a b| (2^-26 typically): less than the rounding of
 // one fp32 product. Each piece product is exact, and one MFMA adds 16 of them
-// per rounding where v_mfma_f32_32x32x2_f32 adds 2, so the result is no further
-// from the exact product than the fp32 MFMA's. Measured against float64
+// per rounding where v_mfma_f32_32x32x2_f32 adds 2, so sums of dense operands are
+// closer to the exact ones than the fp32 MFMA's. Measured against float64
 // (2-norm, N(0,1) operands): K = 16 3.4e-8 (fp32 MFMA 7.0e-8), K = 576 3.6e-7
 // (4.3e-7), K = 4096 9.9e-7 (1.14e-6); uniform [0,1) operands, K = 4096: 5.3e-7
 // (8.5e-7). The nine-product sum measures the same; big pieces first is worse
 // at small K (8.2e-8 at K = 16).
+// Where most products are zero, that turns: a slice rounds its sums six times
+// however few of its products count, and the bf16 MFMA's rounding is not always to
+// nearest. A row with one non-zero element, correctly rounded on the fp32 MFMA, is
+// off by up to 1.45 units in the last place here (21 % of its outputs not the
+// nearest float, 3.5e-8 for 2.5e-8); with n of 2048 elements non-zero, n = 4 7.7e-8
+// (4.0e-8), n = 64 2.9e-7 (1.45e-7). Products of K < 4 run on the fp32 MFMA; rows
+// of zeros in longer ones are not looked for. Adding each slice up on its own and then
+// to the sums (n = 64: 1.5e-7) took 7 to 14 % more time on the smaller tiles and more
+// registers than the large one has.
 //
 // Why: six v_mfma_f32_32x32x16_bf16 take 192 cycles for the 16 k that take
 // v_mfma_f32_32x32x2_f32 512, and the bf16 MFMA runs beside VALU work (the

@@ -91,6 +91,33 @@ def test_small_tile_routes(hip, layout, M, N):
             assert np.array_equal(got.view(np.uint32), (A * B).view(np.uint32))
 
 
+@pytest.mark.parametrize("N", [260, 2048, 4096])
+def test_one_term_sums(hip, N):
+    """A diagonal matrix times another: each output is one product among zeros. Through the pieces it is off by at
+    most the three piece products left out (2^-24 of it) and, as an MFMA's sum is one of the two floats beside the
+    exact one, a unit in the last place and 2^-29 for the roundings of the smaller pieces."""
+    r = np.random.default_rng(9)
+    d, B = r.standard_normal(N).astype(np.float32), r.standard_normal((N, N), dtype=np.float32)
+    exact = d.astype(np.float64)[:, None] * B
+    got = _run(hip, "nn", np.diag(d), B)
+    ulp = np.spacing(np.abs(exact).astype(np.float32)).astype(np.float64)
+    assert np.all(np.abs(got - exact) <= (2.0 ** -24 + 2.0 ** -29) * np.abs(exact) + ulp)
+
+
+@pytest.mark.parametrize("nz", [2, 7, 64])
+@pytest.mark.parametrize("N", [2048, 4096])
+def test_few_term_sums(hip, nz, N):
+    """Rows with nz elements among zeros: each of the (at most nz) slices that hold them adds six piece products to
+    the sums, each addition off by at most 2^-23 of sum |a b|, and leaves 2^-24 out."""
+    r = np.random.default_rng(nz)
+    A, B = np.zeros((N, N), np.float32), r.standard_normal((N, N), dtype=np.float32)
+    for i in range(192):
+        A[i, r.choice(N, nz, replace=False)] = r.standard_normal(nz)
+    got = _run(hip, "nn", A, B)[:192].astype(np.float64)
+    a = A[:192].astype(np.float64)
+    assert np.all(np.abs(got - a @ B) <= (6 * nz * 2.0 ** -23 + 2.0 ** -24) * (np.abs(a) @ np.abs(B)))
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
 @pytest.mark.parametrize("M,N,K", [(70, 67, 40), (128, 256, 2048), (2048, 2048, 50), (2048, 4096, 50), (4096, 4096, 50)])
 def test_special_values(hip, layout, M, N, K):
