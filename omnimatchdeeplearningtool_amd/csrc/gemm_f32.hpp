@@ -83,9 +83,10 @@ inline GemmPlan planGemmFor(int M, int N, int K, int batch, bool wsOk, long long
         while (s < 64 && t * s < 2 * cus && K / (2 * s) >= 128) s *= 2;
         return small(s);
     }
-    // with one tile per CU already, a split must keep >= 512 of K (1024^3: 24.5 us
-    // unsplit, 22.0 split in two)
-    const int minK = t >= cus ? 512 : 256;
+    // with one tile per CU already, a split must keep >= 1024 of K: shorter ones gain
+    // little (1024^3 22.1 us unsplit, 21.3 split in two), and a split needs a workspace, which
+    // a stream that records a graph cannot grow
+    const int minK = t >= cus ? 1024 : 256;
     while (s < 64 && t * s < 2 * cus && K / (2 * s) >= minK) s *= 2;
     return small(s);
 }

@@ -28,6 +28,11 @@ static void check(int M, int N, int K, int batch, long long cus) {
             ++g_fail;
         }
     }
+    const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
+    if (small >= cus && K < 2048 && omhip::planGemmFor(M, N, K, batch, true, cus).splits != 1) {
+        std::printf("FAIL M=%d N=%d K=%d batch=%d cus=%lld: a split where every CU has a tile\n", M, N, K, batch, cus);
+        ++g_fail;
+    }
     // the wsOk rule of gemmF32: 64 splits of the batch's C within 256 MiB
     const bool wsOk = (long long)64 * batch * M * N * 4 <= (256LL << 20);
     const omhip::GemmPlan p = omhip::planGemmFor(M, N, K, batch, wsOk, cus);

@@ -188,6 +188,26 @@ def test_capture_refuses_new_workspace_and_tables(hip, streams):
         g2.destroy()
 
 
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (1000, 1500, 2047)])
+def test_capture_of_products_without_workspace(hip, streams, m, n, k):
+    """A product whose tiles give every CU one and whose K is below 2048 needs no workspace: it is captured on a
+    fresh stream before any eager run, and replays give the eager run's bits."""
+    H = hip.HIPBackend
+    a, b = to_dev(hip, O.randn((m, k), 75)), to_dev(hip, O.randn((k, n), 76))
+    c, c_ref = empty_dev(hip, (m, n)), empty_dev(hip, (m, n))
+    s = streams.create()
+    hip.set_stream(s)
+    g = hip.Graph(lambda: H.matmul(a, b, c, m, k, n))
+    try:
+        H.matmul(a, b, c_ref, m, k, n)
+        for _ in range(2):
+            g.launch()
+            streams.sync(s)
+            assert np.array_equal(_bits(c.numpy()), _bits(c_ref.numpy()))
+    finally:
+        g.destroy()
+
+
 def test_free_on_one_stream_reuse_on_another(hip, streams):
     """A buffer freed on stream A while A's GEMM still reads it must not be handed to stream B:
     B's first split-K GEMM (128x4096x4096, 8 MiB of partials: a fresh workspace block of the
