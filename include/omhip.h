@@ -204,9 +204,11 @@ int omHipMergeHeads(const float* pIn, float* pOut, int nBatch, int nSeqLen, int 
  * tensorBatchedMatmul (Q K^T), tensorSoftmaxLastDim, tensorBatchedMatmul (P V),
  * mergeHeads. pQKV [nBatch*nSeq, 3*D] -> pOut [nBatch*nSeq, D], both fp32. Q is scaled as
  * qkvSplitHeads scales it and products accumulate in fp32. Head dimensions that are multiples
- * of 4 up to 128 run as one kernel without intermediates (running maximum over the keys);
- * others as strided products that read the heads where they lie and omHipSoftmax, with
- * intermediates in the stream's staging workspace. */
+ * of 4 up to 128 run as one kernel without intermediates (running maximum over the keys) unless
+ * few, long heads would leave most of the card idle; those and other head dimensions run as
+ * strided products that read the heads where they lie and omHipSoftmax, with intermediates in
+ * the stream's staging workspace (where that cannot be had, head dimensions of the first kind
+ * run as one kernel all the same). */
 int omHipAttention(const float* pQKV, float* pOut, int nBatch, int nSeq, int nHeads, int nHeadDim, float fScale);
 
 /* ===== fp32 GEMM (cuda_kernels.cuh:109-117) ===== */

@@ -38,7 +38,7 @@ namespace {
 typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
 
 constexpr int kKeys = 64;      // keys per trip
-constexpr int kQueries = 64;   // queries per workgroup, 16 per wave
+constexpr int kQueries = kAttnF32Queries;   // queries per workgroup, 16 per wave
 constexpr int kThreads = 256;
 
 struct AttnF32Params {
@@ -201,10 +201,7 @@ int launchAttnF32(const AttnF32Params& p, int blocks) {
 }  // namespace
 
 bool attentionF32Fits(int B, int S, int H, int hd) {
-    const long long blocks = (long long)B * H * ((S + kQueries - 1) / kQueries);
-    // A workgroup walks all keys of its head alone (about 3 us per 64): beyond 512 keys that pays only where
-    // every CU has a workgroup; the composed path's products spread a few long heads over the card.
-    if (S > 512 && blocks < cuCount()) return false;
+    const long long blocks = (long long)B * H * (((long long)S + kQueries - 1) / kQueries);
     // 16-byte loads of four d; a tile's rows in one buffer view
     return hd % 4 == 0 && hd <= kAttnF32MaxHeadDim && blocks <= 0x7fffffffLL &&
            3LL * H * hd * 4 * kKeys <= (long long)kMaxBufferBytes;
@@ -217,7 +214,7 @@ int attentionF32(const float* qkv, float* out, int B, int S, int H, int hd, floa
     p.S = S;
     p.H = H;
     p.hd = hd;
-    p.qBlocks = (S + kQueries - 1) / kQueries;
+    p.qBlocks = (int)(((long long)S + kQueries - 1) / kQueries);
     p.ldq = 3LL * H * hd;
     p.ldo = (long long)H * hd;
     p.scale = scale;

@@ -297,12 +297,19 @@ int omHipAttention(const float* pQKV, float* pOut, int nBatch, int nSeq, int nHe
     const int outer = headsOuter ? nHeads : nBatch, inner = headsOuter ? nBatch : nHeads;
     if ((long long)inner * S * S > 0x7fffffffLL)
         return fail("%s: %d x %lld x %lld scores exceed the 2^31-element limit", name, inner, S, S);
-    // One kernel wherever it fits (ViT-B/16 b16: 250 us below, 32 us there); the rest takes products of any sizes.
-    if (attentionF32Fits(nBatch, nSeq, nHeads, nHeadDim))
-        return attentionF32(pQKV, pOut, nBatch, nSeq, nHeads, nHeadDim, fScale);
+    // One kernel, or products of any sizes spread over the card. Where those cannot have their workspaces (out of
+    // memory, or a stream that records a graph before its first eager run), the one kernel again, which needs none.
+    const bool fits = attentionF32Fits(nBatch, nSeq, nHeads, nHeadDim);
+    auto fused = [&] { return attentionF32(pQKV, pOut, nBatch, nSeq, nHeads, nHeadDim, fScale); };
+    if (fits && attentionF32Faster(nBatch, nSeq, nHeads, nHeadDim, cuCount())) return fused();
+    auto orFused = [&] {
+        if (!fits) return -1;   // the cause is recorded
+        clearError();
+        return fused();
+    };
     const size_t bQ = up((size_t)(T * D) * 4), bScores = up((size_t)inner * S * S * 4);
     char* base = static_cast<char*>(workspace(bQ + bScores, kWsStaging));
-    if (!base) return -1;   // workspace() recorded the cause
+    if (!base) return orFused();
     float* q = reinterpret_cast<float*>(base);
     float* scores = reinterpret_cast<float*>(base + bQ);
     const long long ldq = 3 * D;
@@ -320,11 +327,11 @@ int omHipAttention(const float* pQKV, float* pOut, int nBatch, int nSeq, int nHe
         float* C = pOut + (headsOuter ? o * Dh : o * S * D);
         if (omHipGemmStridedBatched(0, 1, inner, nSeq, nSeq, nHeadDim, Q, D, innerQ, K, ldq, innerKV, scores, S,
                                     S * S))
-            return -1;
-        if (omHipSoftmax(scores, scores, inner * nSeq, nSeq)) return -1;
+            return orFused();
+        if (omHipSoftmax(scores, scores, inner * nSeq, nSeq)) return orFused();
         if (omHipGemmStridedBatched(0, 0, inner, nSeq, nHeadDim, nSeq, scores, S, S * S, V, ldq, innerKV, C, D,
                                     innerC))
-            return -1;
+            return orFused();
     }
     return 0;
 }

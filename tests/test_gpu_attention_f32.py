@@ -11,12 +11,15 @@ import pytest
 
 import oracle as O
 from conftest import empty_dev, to_dev
+from test_gpu_streams import streams  # noqa: F401  (fixture: caller-owned streams)
 
 pytestmark = pytest.mark.gpu
 
 # S: one key, around 16 and 64, several trips; D: each padded width, the largest, the composed path (10, 132)
 SHAPES = [(2, s, 2, 64) for s in (1, 15, 16, 17, 63, 64, 65, 129, 300)] + \
-         [(1, s, 3, d) for d in (4, 12, 16, 20, 32, 48, 80, 96, 100, 128, 10, 132) for s in (17, 70)]
+         [(1, s, 3, d) for d in (4, 12, 16, 20, 32, 48, 80, 96, 100, 128, 10, 132) for s in (17, 70)] + \
+         [(1, 384, 3, 64), (1, 449, 3, 64), (3, 500, 1, 64), (1, 512, 12, 64), (1, 700, 2, 32), (2, 577, 3, 80),
+          (1, 1000, 12, 20), (2, 1030, 1, 64), (4, 520, 9, 128)]   # both sides of the line between the two paths
 
 
 def _run(hip, qkv, B, S, H, D, scale, shift=0):
@@ -41,6 +44,32 @@ def test_edges(hip, B, S, H, D):
     got = _run(hip, qkv, B, S, H, D, scale, shift=S % 2)
     ref, bound = O.attention_f64(qkv, B, S, H, D, scale)
     assert O.normalized_error(got, ref, bound) <= _tolerance(qkv, B, S, H, D, scale)
+
+
+def test_cold_capture(hip, streams):
+    """Long, few heads take products with intermediates; a fresh stream that records a graph cannot allocate them
+    and records the fused kernel, for the staging array as for the products' own workspace."""
+    B, S, H, D = 1, 1024, 1, 64
+    qkv = O.randn((B * S, 3 * H * D), 13, 1.0)
+    scale = float(np.float32(D ** -0.5))
+    ref, bound = O.attention_f64(qkv, B, S, H, D, scale)
+    dq = to_dev(hip, qkv)
+    s = streams.create()
+    hip.set_stream(s)
+    for warm in (None, (1, 1100, 1, 10)):   # nothing, or another call's staging array alone
+        if warm:
+            b, n, h, d = warm
+            hip.HIPBackend.attention(to_dev(hip, np.zeros((b * n, 3 * h * d), np.float32)), empty_dev(hip, (b * n, h * d)), *warm, 1.0)
+        dout = empty_dev(hip, (B * S, H * D))
+        g = hip.Graph(lambda: hip.HIPBackend.attention(dq, dout, B, S, H, D, scale))
+        try:
+            for _ in range(2):
+                g.launch()
+                streams.sync(s)
+                got = dout.numpy()
+                assert O.normalized_error(got, ref, bound) <= _tolerance(qkv, B, S, H, D, scale)
+        finally:
+            g.destroy()
 
 
 def test_negative_scale_and_large_scores(hip):
