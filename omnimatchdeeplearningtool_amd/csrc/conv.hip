@@ -357,13 +357,14 @@ __device__ __forceinline__ void storeEpilogue(const ConvParams& p, const f32x16 
 // (split-K) writes its partial tile to slot [part][tile] in the registers' own
 // order (16-byte words, consecutive lanes consecutive); then the block counts
 // itself in at the tile's counter, and the block that arrives last adds every
-// part's partials in part order (0 + part 0 + part 1 + ..., kAhead parts in
-// flight), applies the epilogue, writes the output and returns the counter to
+// part's partials in part order (0 + part 0 + part 1 + ..., the loads of kAhead
+// parts issued together as far as registers reach), applies the epilogue, writes the output and returns the counter to
 // zero. One element at a time in [Cout][Nq] order (a dword store and a load that
 // is waited for per element and part) the hand-over was a chain of memory
 // latencies at the end of every split layer: ResNet-18 on one image 336 -> 284 us,
-// a 5x5 stride-2 layer of 5 images 46 x 61 x 53 -> 75 channels 21.9 -> 20.1 us, the
-// convolutions of 32 images 1106 -> 1096 us. The order of
+// a 5x5 stride-2 layer of 5 images 46 x 61 x 53 -> 75 channels 21.9 -> 20.1 us; the
+// convolutions of 32 images, where few blocks are last, are the same within the runs'
+// differences. The order of
 // the sum does not depend on which block arrives last, so the result is
 // deterministic and equal to a separate finishing pass's. Partials are
 // written and read with agent-coherent (sc1) accesses — the encoding of
@@ -634,7 +635,12 @@ struct ConvPlan {
 //  * Fewer than 2 tiles per CU (late ResNet stages: few pixels, many
 //    channels): split K uniformly by the s in [1, 16] (>= 128 taps per split)
 //    that minimises ceil(tiles*s/CUs)/s tile-times per CU plus s extra fp32
-//    writes and reads of the output (e.g. 512x1568x4608: 5 splits).
+//    writes and reads of the output (e.g. 512x1568x4608: 5 splits). What moves is
+//    whole tiles, up to eight times the output where it has few channels; a plan
+//    that counts those was faster for some such layers and slower for more, us: 32 images
+//    128 x 28 x 28 -> 8 channels 41.0 -> 37.1, 20 images 128 x 30 x 30 -> 16 33.9 -> 30.0, but
+//    18 images 224 x 24 x 35 -> 9 46.9 -> 60.6, 32 images 64 x 28 x 28 -> 8 22.1 -> 25.7, 1 image
+//    160 x 68 x 68 -> 8 16.9 -> 19.9 (the partials stay in the caches).
 //  * Otherwise, when the tile count is not a multiple of the CU count and the
 //    CUs hold few tiles each: the tiles beyond the last whole round run as K
 //    pieces (one per idle CU, at most 16 per tile), summed by each tile's last
@@ -650,7 +656,7 @@ static ConvPlan planConv(const ConvParams& p, bool haveSplitWs) {
     if (T < 2 * U) {
         if (!haveSplitWs) return pl;
         // seconds: one tile on one CU at 65 % of its share of peak; one split's partial
-        // write + read at an effective 6 TB/s (it partly overlaps the MFMA work)
+        // write + read of the output's size at an effective 6 TB/s (it partly overlaps the MFMA work)
         const double tileT = 2.0 * Cfg::BM * Cfg::BN * p.K / (0.65 * 157.3e12 / 256.0);
         const double partT = 8.0 * p.Cout * (double)p.Nq / 6.0e12;
         double best = (double)((T + U - 1) / U) * tileT;
