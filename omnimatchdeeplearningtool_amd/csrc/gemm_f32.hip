@@ -653,7 +653,7 @@ static int linearBackward(const float* X, const float* G, const float* W, const 
     using Plain = std::integral_constant<Path, Path::Plain>;
     using Far = std::integral_constant<Path, Path::Far>;
     if (!views) return launch(Far{}, Far{});
-    const bool plainW = smallTilePlain(tilesW, B, B, true, false, cuCount()), plainX = !dX || smallTilePlain(tilesX, O, O, false, true, cuCount());
+    const bool plainW = smallTilePlain(tilesW, B, B, true, false, I % 4 || O % 4, cuCount()), plainX = !dX || smallTilePlain(tilesX, O, O, false, true, false, cuCount());
     if (plainW) return plainX ? launch(Plain{}, Plain{}) : launch(Plain{}, Pieces{});
     return plainX ? launch(Pieces{}, Plain{}) : launch(Pieces{}, Pieces{});
 }

@@ -33,14 +33,18 @@ inline int splitPieces(int K, int splits, int* kChunk = nullptr) {
 //     9.8 / 8.5, 11.0 / 8.6; 1024x1024x256 8.3 / 8.1, 8.2 / 7.9, 9.1 / 8.2; x1000 23.1 / 22.1, 22.7 / 21.3, 25.9 / 22.4;
 //   split: 128x256x784 10.3 / 10.0, 10.8 / 9.9, 11.1 / 10.0; 256x256x512 8.5 / 8.9, 9.1 / 8.8, 9.1 / 8.9; x4096 (16
 //     pieces) 17.4 / 18.9, 19.4 / 18.8, 18.2 / 19.5; 8x4096x4096 (pieces of 512) 21.8 / 25.1, 23.0 / 24.8, 23.9 / 25.6;
-//     87x108x3284 (of 416) 15.0 / 15.5, 15.9 / 15.2, 16.3 / 15.6;
+//     87x108x3284 (of 416) 15.0 / 15.5, 15.9 / 15.2, 16.3 / 15.6; 19x1212x1160 (of 304)
+//     12.7 / 12.1, 12.8 / 11.9, 13.9 / 13.1; 128x4000x2100 TN (8 of 272, 1008 workgroups) 28.6 / 25.8;
 //   more tiles than CUs: 1024x2048x64 6.8 / 6.4, x100 9.1 / 8.0, x160 9.5 / 9.3, x256 11.6 / 12.2; 600 of 64x64x32
 //     7.8 / 6.4, x128 13.1 / 11.2.
-constexpr bool smallTilePlain(long long tiles, int K, int chunk, bool ta, bool tb, long long cus) {
+// Rows of an operand stored K first that are no multiple of four (`ragged`) load element by element there.
+constexpr bool smallTilePlain(long long tiles, int K, int chunk, bool ta, bool tb, bool ragged, long long cus) {
     if (tiles > cus) return K <= (K % 32 ? 320 : 192);
+    if (ragged && chunk > 320) return false;
     if (chunk >= K) return true;
-    if (tb && !ta) return chunk < 512;
-    return chunk <= 256 && (ta ? K < 2048 : chunk % 32 != 0);
+    if (chunk >= 512) return false;
+    if (tiles * ((K + chunk - 1) / chunk) > 2 * cus) return true;   // the pieces' LDS holds two workgroups per CU
+    return tb && !ta ? true : K < 2048 && (ta || chunk % 32 != 0);
 }
 
 // Tile and split-K choice on a device of `cus` compute units. A launch takes as
@@ -70,7 +74,8 @@ inline GemmPlan planGemmFor(int M, int N, int K, int batch, bool wsOk, long long
     auto small = [&](int splits) {
         int chunk;
         splitPieces(K, splits, &chunk);
-        return GemmPlan{2, splits, smallTilePlain(t, K, chunk, ta, tb, cus)};
+        const bool ragged = (ta && M % 4) || (!tb && N % 4);
+        return GemmPlan{2, splits, smallTilePlain(t, K, chunk, ta, tb, ragged, cus)};
     };
     if (K < 4 || (K <= 32 && t <= 4 * cus) || (K <= 128 && tiles(128, 128) < cus)) return small(1);
     const double costL = 2.25 * rounds(tiles(256, 256)), costM = 0.66 * rounds(tiles(128, 128));

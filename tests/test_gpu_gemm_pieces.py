@@ -76,7 +76,8 @@ def test_tile_edges(hip, layout, M, N):
 ROUTES = [(64, 60, k) for k in (1, 2, 3, 4, 5, 19, 31, 32, 33, 36, 511, 512, 530, 1000, 1023, 1024, 1030, 2047, 2048, 4100)] + \
          [(61, 131, k) for k in (1, 3, 18, 47, 512, 1023, 1025, 2050)] + [(9, 4096, k) for k in (2040, 4099)] + \
          [(1000, 2047, k) for k in (1, 30, 33, 191, 192, 193, 224, 288, 319, 320, 321, 322, 323, 338, 352)] + \
-         [(1500, 1501, k) for k in (32, 33, 127, 128, 129)]
+         [(1500, 1501, k) for k in (32, 33, 127, 128, 129)] + \
+         [(100, 1000, k) for k in (1100, 1216, 1500, 2100)] + [(128, 4000, 2100), (333, 999, 321), (333, 999, 319)]
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
