@@ -231,7 +231,7 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
             mmaSplitSub<Cfg, SUB, SIDES, kSideValu>(cur, cur + OFF_B, SLICE, acc[0][0], wm, wn, lane, side);
         else
             mmaSplitSlice<Cfg, SIDES, kSideValu>(cur, cur + OFF_B, acc, wm, wn, lane, [&](int i) { side(0, i); });
-        __syncthreads();
+        if (FULL || T + 1 < nt) __syncthreads();   // after the last stage the tile's vote is the barrier
     };
     // Stages 0 and 1 are loaded together (one memory latency before the first products, not
     // two). The main loop's own first loads test nothing: its waits then count the same loads
@@ -283,13 +283,14 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
 // the buffer views).
 enum class Path { Pieces, Plain, Far };
 
-// LDS: two stages of both operands' slices, as pieces or as they are; a tile of
-// the pieces that is computed again uses its stages for the plain slices.
+// LDS: two stages of both operands' slices, as pieces (and a word per wave behind
+// them, its vote on non-finite sums) or as they are; a tile of the pieces that is
+// computed again uses its stages for the plain slices.
 template <class Cfg, Path PATH>
 constexpr size_t ldsBytes() {
     constexpr size_t plain = sizeof(float) * (LdsShape<Cfg::BM, 16>::SIZE + LdsShape<Cfg::BN, 16>::SIZE);
     static_assert(kSliceBytes<Cfg> >= plain);
-    return 2 * (PATH == Path::Pieces ? kSub<Cfg> * kSliceBytes<Cfg> : plain);
+    return PATH == Path::Pieces ? 2 * kSub<Cfg> * kSliceBytes<Cfg> + Cfg::NWAVES * sizeof(int) : 2 * plain;
 }
 
 // One output tile (bid: the tile's linear index, batch, split) of C =
@@ -372,17 +373,16 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
         plain();
     } else {
         splitLoop<Cfg, TA, TB>(p, smem, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
-        int* const bad = reinterpret_cast<int*>(smem);   // a word per wave; the stages are free
+        // behind the stages, which other waves may still read: one barrier ends the main loop and the vote
+        // (1001 x 765 x 1537 TN with a barrier of its own 29.05 us, so 28.85)
+        int* const bad = reinterpret_cast<int*>(smem + 2 * kSub<Cfg> * kSliceBytes<Cfg>);
         const bool mine = __any(unscaleSums(acc));
         if (lane == 0) bad[wave] = mine;
         __syncthreads();
         int any = 0;
 #pragma unroll
         for (int w = 0; w < Cfg::NWAVES; ++w) any |= bad[w];
-        if (__builtin_amdgcn_readfirstlane(any)) {
-            __syncthreads();
-            plain();
-        }
+        if (__builtin_amdgcn_readfirstlane(any)) plain();
     }
 
     const int li = lane & 31, h = lane >> 5;
