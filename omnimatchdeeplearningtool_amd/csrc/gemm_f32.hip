@@ -382,7 +382,9 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
         int any = 0;
 #pragma unroll
         for (int w = 0; w < Cfg::NWAVES; ++w) any |= bad[w];
-        if (__builtin_amdgcn_readfirstlane(any)) plain();
+        // laid out behind the epilogue: a jump over its 600 instructions at the end of every tile cost
+        // 128 x 4096 x 4096 0.1 us of 36.6 and 1001 x 765 x 1537 TN 0.4 of 30
+        if (__builtin_amdgcn_readfirstlane(any)) [[unlikely]] plain();
     }
 
     const int li = lane & 31, h = lane >> 5;
