@@ -231,7 +231,7 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
             mmaSplitSub<Cfg, SUB, SIDES, kSideValu>(cur, cur + OFF_B, SLICE, acc[0][0], wm, wn, lane, side);
         else
             mmaSplitSlice<Cfg, SIDES, kSideValu>(cur, cur + OFF_B, acc, wm, wn, lane, [&](int i) { side(0, i); });
-        if (FULL || T + 1 < nt) __syncthreads();   // after the last stage the tile's vote is the barrier
+        __syncthreads();
     };
     // Stages 0 and 1 are loaded together (one memory latency before the first products, not
     // two). The main loop's own first loads test nothing: its waits then count the same loads
@@ -283,14 +283,13 @@ __device__ __forceinline__ void splitLoop(const GemmF32Params& p, char* smem, f3
 // the buffer views).
 enum class Path { Pieces, Plain, Far };
 
-// LDS: two stages of both operands' slices, as pieces (and a word per wave behind
-// them, its vote on non-finite sums) or as they are; a tile of the pieces that is
-// computed again uses its stages for the plain slices.
+// LDS: two stages of both operands' slices, as pieces or as they are; a tile of
+// the pieces that is computed again uses its stages for the plain slices.
 template <class Cfg, Path PATH>
 constexpr size_t ldsBytes() {
     constexpr size_t plain = sizeof(float) * (LdsShape<Cfg::BM, 16>::SIZE + LdsShape<Cfg::BN, 16>::SIZE);
     static_assert(kSliceBytes<Cfg> >= plain);
-    return PATH == Path::Pieces ? 2 * kSub<Cfg> * kSliceBytes<Cfg> + Cfg::NWAVES * sizeof(int) : 2 * plain;
+    return 2 * (PATH == Path::Pieces ? kSub<Cfg> * kSliceBytes<Cfg> : plain);
 }
 
 // One output tile (bid: the tile's linear index, batch, split) of C =
@@ -373,9 +372,7 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
         plain();
     } else {
         splitLoop<Cfg, TA, TB>(p, smem, acc, m0, n0, batch, kBeg, kEnd, wm, wn, lane, tid);
-        // behind the stages, which other waves may still read: one barrier ends the main loop and the vote
-        // (1001 x 765 x 1537 TN with a barrier of its own 29.05 us, so 28.85)
-        int* const bad = reinterpret_cast<int*>(smem + 2 * kSub<Cfg> * kSliceBytes<Cfg>);
+        int* const bad = reinterpret_cast<int*>(smem);   // a word per wave; the stages are free
         const bool mine = __any(unscaleSums(acc));
         if (lane == 0) bad[wave] = mine;
         __syncthreads();
@@ -383,8 +380,11 @@ __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, 
 #pragma unroll
         for (int w = 0; w < Cfg::NWAVES; ++w) any |= bad[w];
         // laid out behind the epilogue: a jump over its 600 instructions at the end of every tile cost
-        // 128 x 4096 x 4096 0.1 us of 36.6 and 1001 x 765 x 1537 TN 0.4 of 30
-        if (__builtin_amdgcn_readfirstlane(any)) [[unlikely]] plain();
+        // 1001 x 765 x 1537 TN 0.6 us of 29.8 (128 x 4096 x 4096 and 4096^3: nothing)
+        if (__builtin_amdgcn_readfirstlane(any)) [[unlikely]] {
+            __syncthreads();
+            plain();
+        }
     }
 
     const int li = lane & 31, h = lane >> 5;
