@@ -299,10 +299,11 @@ constexpr size_t ldsBytes() {
 // MFMA, whole, so the last bits of its finite elements depend on such neighbours
 // (and on which tile the plan chose); where all sums of a tile are finite, every
 // tile adds a product's terms in the same order.
-// Computing again costs that unit's time after the pieces': 4096^3 with one NaN
-// element 1489 us, with NaN in every element 1379 (563 without, 952 on the fp32
-// MFMA alone); 1024^3 26.8 and 36.5 (20.8; 22.4). Read from memory by each wave
-// for its own block, without LDS, it took 3385, 5309, 58 and 91.
+// Computing again costs that unit's time after the pieces', us, finite / one NaN
+// element / all NaN: 4096^3 568 / 1465 / 1352 (952 on the fp32 MFMA alone), 2048^3
+// 106 / 217 / 213, 128 x 4096 x 4096 41.6 / 55 / 64; 1024^3 runs on the fp32 MFMA
+// anyway. Read from memory by each wave for its own block, without LDS, 4096^3 took
+// 3385 and 5309.
 template <class Cfg, bool TA, bool TB, Path PATH, bool GATE = false>
 __device__ __forceinline__ void gemmF32Tile(const GemmF32Params& p, char* smem, int bid, long long batch, int split) {
     static_assert(Cfg::BK == 16, "one MFMA step per slice");
@@ -457,7 +458,7 @@ static bool splitViewOk(bool kMajor, int R, int rows, long long ld) {
 // The large tile runs 8 waves of 64 x 128 (two per SIMD, 128 accumulators
 // each): while one wave splits its share of the next slice or waits on its
 // fragment reads and the block barrier, the other keeps the matrix core busy.
-// It is bound by power: 4096^3 takes 570-605 us (227-241 TFLOP/s = 1.36-1.45
+// It is bound by power: 4096^3 takes 551-605 us (227-249 TFLOP/s = 1.36-1.50
 // PFLOP/s of bf16 MFMA, what a library bf16 product of 8192^3 reaches on this
 // card, 1.37); on the fp32 MFMA it took 951-961 us (0.92 of that unit's peak).
 // Beside it: 8192^3 7.49 -> 4.74 ms, 3072^3 (128x128 tiles) 538 -> 345 us, 2048^3
